@@ -112,7 +112,8 @@ struct GemmTile {
 // Tile the launcher would use for this shape ({-1,-1} when no M tile divides
 // the relay tile). coresident: skip 256x256, whose four waves take every
 // register of the CU (a workgroup of a concurrently spinning consumer would
-// otherwise keep the CU from the GEMM).
-GemmTile GemmPickTile(int M, int N, int relay_rows, bool coresident = false);
+// otherwise keep the CU from the GEMM). K: the depth of the product (the
+// choice without a relay depends on it).
+GemmTile GemmPickTile(int M, int N, int relay_rows, bool coresident = false, int K = 4096);
 
 }  // namespace kr

@@ -298,6 +298,20 @@ __device__ void TailSwiglu(const GemmParams &p)
     }
 }
 
+// A split tile's finisher arrives on every relay tile that its rows m0 ..
+// m0 + bm - 1 touch; a relay tile is released by the finishers of the row
+// blocks that touch it, in every column.
+__device__ __forceinline__ void ArriveRows(const GemmParams &p, int m0, int bm)
+{
+    if (p.pub.ctrl == nullptr) return;
+    RelayPub pub = p.pub;
+    const int R = pub.rows_per_tile;
+    for (int r = m0 / R; r * R < min(m0 + bm, p.M); ++r) {
+        pub.arrivals = ((min(r * R + R, p.M) - 1) / bm - r * R / bm + 1) * p.tiles_n;
+        RelayArrive(pub, r);
+    }
+}
+
 // ------------------------------------------- Add+RMSNorm relay consumer
 // The producer's own workgroups consume its released row tiles (the
 // reference's down -> Add+RMSNorm tile loop, exec/qwen_main.cpp:1274-1302,
@@ -374,6 +388,24 @@ __device__ void NormTail(const GemmParams &p, int tile, int worker, int workers)
             StoreRelaxed(flag + kOffStatus, to ? 2 : 1);
         }
     }
+}
+
+// The Add+RMSNorm relay consumer of a split grid (G workgroups, all resident):
+// after its own pieces each workgroup takes a share of one relay tile (of
+// every G-th, should the tiles outnumber the workgroups). A share of every
+// tile in turn had each workgroup wait, load and count once per relay tile:
+// 768x4096x4096 in four relay tiles 65 us, 768x3584x18944 155.
+template <int DT, int NW, int WPE>
+__device__ __forceinline__ void NormTailShare(const GemmParams &p, int G)
+{
+    const int tiles = p.M / p.pub.rows_per_tile, b = int(blockIdx.x);
+    int t = b, first = b, next = b + 1;  // workgroups first .. next - 1 work on tile t
+    if (tiles < G) {
+        t = ((b + 1) * tiles - 1) / G;
+        first = t * G / tiles;
+        next = (t + 1) * G / tiles;
+    }
+    for (; t < tiles; t += G) NormTail<DT, NW, WPE>(p, t, b - first, next - first);
 }
 
 // The unary consumer's pass over the staged tile (after C's): y = f(C) with
@@ -643,7 +675,7 @@ __device__ __forceinline__ void StageSwiglu(f32x4 (&acc)[MI][NI][4], uint16_t *s
 {
     constexpr int AW = BN / 2;  // act columns of the tile
     constexpr int WTA = NI * 16;  // act columns per wave
-    static_assert(AW >= 128, "slot swizzle needs >= 32 slots per row");
+    constexpr int SM = AW / 4 - 1 < 31 ? AW / 4 - 1 : 31;  // the slots of a row the swizzle spans
     const int lr = lane & 15;
     const int hi = lane >> 5;                // after the swap: sub-block rows 16 hi ..
     const int lc = 4 * ((lane >> 4) & 1);    // first act column of the lane in its group
@@ -665,7 +697,7 @@ __device__ __forceinline__ void StageSwiglu(f32x4 (&acc)[MI][NI][4], uint16_t *s
                     const float u = RoundTo<DT>(__uint_as_float(sw[1]));
                     h[e] = Elem<DT>::Store(RoundTo<DT>(Silu(g)) * u);
                 }
-                const int slot = (acol >> 2) ^ (row & 31);
+                const int slot = (acol >> 2) ^ (row & SM);
                 *reinterpret_cast<uint2 *>(stage + row * AW + slot * 4) =
                     make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
             }
@@ -681,7 +713,7 @@ __device__ __forceinline__ void StageSwiglu(f32x16 (&acc)[MI][NI], uint16_t *sta
 {
     constexpr int AW = BN / 2;  // act columns of the tile
     constexpr int WTA = NI * 16;  // act columns per wave
-    static_assert(AW >= 128, "slot swizzle needs >= 32 slots per row");
+    constexpr int SM = AW / 4 - 1 < 31 ? AW / 4 - 1 : 31;  // the slots of a row the swizzle spans
     const int lrow = lane & 31;
     const int lhalf = lane >> 5;
 #pragma unroll
@@ -699,7 +731,7 @@ __device__ __forceinline__ void StageSwiglu(f32x16 (&acc)[MI][NI], uint16_t *sta
                     const float u = RoundTo<DT>(acc[i][j][8 * q + 4 + e]);
                     h[e] = Elem<DT>::Store(RoundTo<DT>(Silu(g)) * u);
                 }
-                const int slot = (acol >> 2) ^ (row & 31);
+                const int slot = (acol >> 2) ^ (row & SM);
                 *reinterpret_cast<uint2 *>(stage + row * AW + slot * 4) =
                     make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
             }
@@ -715,6 +747,7 @@ __device__ __forceinline__ void StoreTileSwiglu(const GemmParams &p, ACC &acc, u
     StageSwiglu<DT, BM, BN>(acc, stage, wm, wn, lane);
     __syncthreads();
     constexpr int CPR = AW / 8;
+    constexpr int SM = AW / 4 - 1 < 31 ? AW / 4 - 1 : 31;
     const int64_t a0 = n0 / 2;
     const int acols = p.N / 2;
 #pragma unroll 4
@@ -724,7 +757,7 @@ __device__ __forceinline__ void StoreTileSwiglu(const GemmParams &p, ACC &acc, u
         const int gm = m0 + row;
         const int gn = int(a0) + ch * 8;
         if (gm >= p.M || gn >= acols) continue;
-        uint4 v = *reinterpret_cast<const uint4 *>(stage + row * AW + (ch ^ ((row & 31) >> 1)) * 8);
+        uint4 v = *reinterpret_cast<const uint4 *>(stage + row * AW + (ch ^ ((row & SM) >> 1)) * 8);
         if (row & 1) v = make_uint4(v.z, v.w, v.x, v.y);
         PutU128(p.epi_act + int64_t(gm) * p.ld_act + gn, v, p.store_kind == 0 || p.pub.ctrl != nullptr);
     }
@@ -859,12 +892,8 @@ GemmKernel(GemmParams p)
         __syncthreads();
     }
 
-    if constexpr (BN >= 256) {
-        if (p.epi_act != nullptr) {
-            StoreTileSwiglu<DT, BM, BN, kThreads>(p, acc, smem, m0, n0, wm, wn, lane);
-        } else {
-            StoreTile<DT, BM, BN, kThreads>(p, acc, smem, m0, n0, wm, wn, lane);
-        }
+    if (p.epi_act != nullptr) {
+        StoreTileSwiglu<DT, BM, BN, kThreads>(p, acc, smem, m0, n0, wm, wn, lane);
     } else {
         StoreTile<DT, BM, BN, kThreads>(p, acc, smem, m0, n0, wm, wn, lane);
     }
@@ -993,6 +1022,8 @@ int PrefetchStages()
 // iterations, at most pmax pieces per tile.
 struct StreamKPlan {
     int G = 0, tiles = 0, nk = 0, pmax = 0;
+    int bm = 256, bn = 256;  // below 256 rows: GemmSplitKernel, every tile in G / tiles pieces
+    size_t WsBytes() const { return size_t(tiles) * pmax * bm * bn * 4; }
 };
 
 int CuCount()
@@ -1006,14 +1037,22 @@ int CuCount()
     return v;
 }
 
+// Whether a launch of bm x bn tiles has at most one workgroup per CU.
+bool DeepGrid(int bm, int bn, int M, int N)
+{
+    return ((M + bm - 1) / bm) * ((N + bn - 1) / bn) <= CuCount();
+}
+
 using GemmFn = void (*)(GemmParams);
 
 // The kernel a launch of BM x BN tiles runs over K, and its block size: the
 // 8-wave staged kernel for 192x256; for 256x256 the 8-wave kernel (stream-K
 // or data-parallel) unless KR_GEMM_WAVES=4; the 4-wave pipelined kernel for
 // the other tiles; the simple kernel where K % 64 != 0 or KR_GEMM_SIMPLE=1.
+// A small tile whose grid has at most one workgroup per CU takes the deep
+// ring.
 template <int DT, int BM, int BN>
-GemmFn PickGemmKernel(int K, bool sk, int &threads)
+GemmFn PickGemmKernel(int M, int N, int K, bool sk, int &threads)
 {
     if constexpr (BM == 192) {
         // 192x256: the 8-wave staged kernel only (GemmLaunch picks this tile
@@ -1038,6 +1077,9 @@ GemmFn PickGemmKernel(int K, bool sk, int &threads)
                 }
             }
             threads = kThreads;
+            if constexpr (BM * BN < 256 * 128 && BN == 128) {
+                if (DeepGrid(BM, BN, M, N)) return GemmPipeKernel<DT, BM, BN, 0, 4, false, 0, DeepStages<BM, BN>()>;
+            }
             switch (PrefetchStages()) {
             case 2: return GemmPipeKernel<DT, BM, BN, 2, 4>;
             case 4: return GemmPipeKernel<DT, BM, BN, 4, 4>;
@@ -1051,15 +1093,15 @@ GemmFn PickGemmKernel(int K, bool sk, int &threads)
 
 // Workgroups of that kernel one CU holds at once, from the runtime's
 // occupancy query on the exact instantiation (registers, LDS, waves);
-// cached per (dtype, tile, K-path, stream-K).
+// cached per (dtype, tile, K-path, stream-K, ring).
 template <int DT, int BM, int BN>
-int GemmWgsPerCu(int K, bool sk)
+int GemmWgsPerCu(int M, int N, int K, bool sk)
 {
-    static int cache[2][2] = {{-1, -1}, {-1, -1}};
-    int &c = cache[K % kPipeK == 0 ? 1 : 0][sk ? 1 : 0];
-    if (c < 0) {
+    static int cache[2][2][2] = {};  // 0: not asked yet
+    int &c = cache[K % kPipeK == 0][sk][DeepGrid(BM, BN, M, N)];
+    if (c == 0) {
         int threads = 0;
-        const GemmFn fn = PickGemmKernel<DT, BM, BN>(K, sk, threads);
+        const GemmFn fn = PickGemmKernel<DT, BM, BN>(M, N, K, sk, threads);
         int n = 0;
         Check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void *>(fn), threads, 0),
               "gemm occupancy");
@@ -1069,16 +1111,17 @@ int GemmWgsPerCu(int K, bool sk)
     return c;
 }
 
-int GemmWgsPerCu(int dt, int bm, int bn, int K, bool sk)
+int GemmWgsPerCu(int dt, int bm, int bn, int M, int N, int K, bool sk)
 {
     const bool bf = dt == kBF16;
 #define KR_OCC_CASE(BM_, BN_) \
-    if (bm == BM_ && bn == BN_) return bf ? GemmWgsPerCu<kBF16, BM_, BN_>(K, sk) : GemmWgsPerCu<kF16, BM_, BN_>(K, sk);
+    if (bm == BM_ && bn == BN_) return bf ? GemmWgsPerCu<kBF16, BM_, BN_>(M, N, K, sk) : GemmWgsPerCu<kF16, BM_, BN_>(M, N, K, sk);
     KR_OCC_CASE(256, 256)
     KR_OCC_CASE(192, 256)
     KR_OCC_CASE(256, 128)
     KR_OCC_CASE(128, 256)
     KR_OCC_CASE(128, 128)
+    KR_OCC_CASE(64, 128)
     KR_OCC_CASE(64, 256)
 #undef KR_OCC_CASE
     throw std::runtime_error("gemm: unsupported tile " + std::to_string(bm) + "x" + std::to_string(bn));
@@ -1093,13 +1136,127 @@ int GemmWgsPerCu(int dt, int bm, int bn, int K, bool sk)
 // the kernel the launch runs.
 bool NormRelayResident(int dt, int bm, int bn, int M, int N, int K, int rows_per_tile, int sk_wgs)
 {
-    if (sk_wgs > 0) return sk_wgs <= CuCount() * GemmWgsPerCu(dt, 256, 256, K, true);
+    if (sk_wgs > 0 && bm < 256) return sk_wgs <= CuCount();  // GemmSplitKernel: one per CU
+    if (sk_wgs > 0) return sk_wgs <= CuCount() * GemmWgsPerCu(dt, 256, 256, M, N, K, true);
     if (rows_per_tile <= 0 || rows_per_tile % bm != 0 || M % rows_per_tile != 0) return false;
     const int per = (rows_per_tile / bm) * ((N + bn - 1) / bn);
-    return per <= CuCount() * GemmWgsPerCu(dt, bm, bn, K, false);
+    return per <= CuCount() * GemmWgsPerCu(dt, bm, bn, M, N, K, false);
+}
+
+// Estimated time (us) of a 256x256 split in S pieces (the last one sums all
+// partials alone, so the fix-up grows with S).
+double Split256Us(int K, int S)
+{
+    return 21.0 + (K / kPipeK + S - 1) / S * 1.5 + 2.0 * S;
+}
+
+// Estimated time (us) of a product in bm x 128 tiles, one workgroup per CU on
+// the deep ring, each tile in S pieces of K; negative when that does not fit.
+// Fitted to M 37..1500 at the projections of the three shipped models (within
+// 15%): a launch costs 6, a stage 0.24 (64 rows) / 0.32 (128) alone and 0.38 /
+// 0.59 with every CU loading, a fix-up 2 plus 0.5 / 1.4 a piece.
+double SmallTileUs(int bm, int S, int M, int N, int K)
+{
+    const int tiles = ((M + bm - 1) / bm) * ((N + 127) / 128), G = tiles * S, nk = K / kPipeK;
+    if (K % kPipeK != 0 || G > CuCount() || nk < 2 * S) return -1.0;
+    const double load = double(G) / CuCount();
+    const double stage = bm == 64 ? 0.24 + 0.14 * load : 0.32 + 0.27 * load;
+    const double fix = S > 1 ? 2.0 + (bm == 64 ? 0.5 : 1.4) * S : 0.0;
+    return 6.0 + (nk + S - 1) / S * stage + fix;
+}
+
+// Split plan of a small product (GemmSplitKernel): the cheapest of 64 and 128
+// row tiles in up to 16 pieces, taken when it beats the same tiles unsplit and
+// the 256x256 split `big` (its pieces; 0: none). Below 1920 rows only: longer
+// prompts keep the 256x256 plan and its workspace.
+bool PlanSplit(int M, int N, int K, int big, StreamKPlan &pl)
+{
+    if (M >= 1920 || K % kPipeK != 0) return false;
+    double best = big > 1 ? Split256Us(K, big) : 1e30;
+    int bm = 0, S = 0;
+    for (int b : {64, 128}) {
+        for (int s = 1; s <= 16; ++s) {
+            const double us = SmallTileUs(b, s, M, N, K);
+            if (us < 0.0 || us >= best) continue;
+            best = us;
+            bm = b;
+            S = s;
+        }
+    }
+    if (bm == 0) return false;
+    pl.bm = bm;
+    pl.bn = 128;
+    pl.nk = K / kPipeK;
+    pl.tiles = ((M + bm - 1) / bm) * ((N + 127) / 128);
+    pl.pmax = S;
+    pl.G = S * pl.tiles;
+    return true;
+}
+
+// Tile of a launch that releases relay tiles or shares its CUs, or that the
+// estimates below do not cover.
+GemmTile PickRelayTile(int M, int N, int relay_rows, bool coresident)
+{
+    // Candidates from most to least data reuse; take the first that keeps the
+    // device busy (>= 2 full waves of workgroups, or whole waves) or, failing
+    // that, the one with the best wave efficiency. A GEMM whose 128x128 tiles
+    // give every workgroup a CU of its own takes them: with so few workgroups
+    // each CU's load path is the limit, and smaller tiles put more CUs to
+    // work.
+    static const GemmTile cands[] = {{256, 256}, {256, 128}, {128, 256}, {128, 128}, {64, 256}};
+    const int cus = 256;
+    if ((relay_rows == 0 || relay_rows % 128 == 0) && ((M + 127) / 128) * ((N + 127) / 128) <= cus)
+        return {128, 128};
+    GemmTile best{-1, -1};
+    double best_eff = -1.0;
+    for (const GemmTile &t : cands) {
+        if (relay_rows > 0 && relay_rows % t.bm != 0) continue;
+        if (coresident && t.bm * t.bn >= 256 * 256) continue;
+        const int tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+        const int slots = cus * (t.bm * t.bn >= 256 * 128 ? 1 : 2);
+        // enough workgroups for two rounds, or whole rounds exactly
+        if (tiles >= 2 * slots || tiles % slots == 0) return t;
+        const double work = double(t.bm) * t.bn;  // per-workgroup work unit
+        const double eff = double(tiles) * work / (double((tiles + slots - 1) / slots) * slots * work);
+        const double score = eff * (t.bm * t.bn >= 256 * 128 ? 1.0 : 0.85);
+        if (score > best_eff) {
+            best_eff = score;
+            best = t;
+        }
+    }
+    return best;
+}
+
+// Pieces of the 256x256 split (below).
+int Split256Pieces(int M, int N, int tiles, int nk)
+{
+    const GemmTile dp = PickRelayTile(M, N, 0, false);
+    const int dp_tiles = ((M + dp.bm - 1) / dp.bm) * ((N + dp.bn - 1) / dp.bn);
+    const int dp_slots = CuCount() * (dp.bm * dp.bn >= 256 * 128 ? 1 : 2);
+    const int dp_rounds = (dp_tiles + dp_slots - 1) / dp_slots;
+    const double fill = double(dp_tiles) / (double(dp_rounds) * dp_slots);
+    static const bool longk = [] {
+        const char *e = std::getenv("KR_GEMM_SK_LONGK");
+        return e == nullptr || std::atoi(e) != 0;
+    }();
+    static const int longk_nk = [] {
+        const char *e = std::getenv("KR_GEMM_SK_LONGK_NK");
+        return e != nullptr ? std::max(32, std::atoi(e)) : 256;
+    }();
+    if (fill >= 0.6 && !(longk && fill < 0.9 && nk >= longk_nk)) return 0;
+    const int S = std::min(CuCount() / tiles, nk / 16);
+    // 128x128 tiles run one workgroup per CU on the deep ring: where they
+    // fill 60% of the CUs they stay whole unless the split is estimated
+    // faster (4096x1024x4096: 38 us against 57 in four pieces; 1024x3584x18944:
+    // 160 against 137)
+    if (dp.bm == 128 && dp.bn == 128 && dp_tiles >= 0.6 * CuCount() && dp_tiles <= CuCount() &&
+        SmallTileUs(128, 1, M, N, nk * kPipeK) < Split256Us(nk * kPipeK, std::max(S, 1)))
+        return 0;
+    return S;
 }
 
 // Stream-K plan of a GEMM whose data-parallel tiling leaves CUs idle.
+// Small products first: see PlanSplit. Otherwise:
 // Default: an exact split of K over 256x256 tiles, S = CUs / tiles pieces per
 // tile, each piece at least 16 K stages (S >= 2), so every workgroup runs one
 // piece and the workgroups of an XCD walk K in step on a compact patch of
@@ -1119,28 +1276,22 @@ bool NormRelayResident(int dt, int bm, int bn, int M, int N, int K, int rows_per
 // even spread over G workgroups (a measurement aid).
 bool PlanStreamK(int M, int N, int K, StreamKPlan &pl)
 {
-    if (K % kPipeK != 0 || M < 256 || N < 256) return false;
+    pl = StreamKPlan{};
+    if (K % kPipeK != 0) return false;
     pl.tiles = ((M + 255) / 256) * ((N + 255) / 256);
     pl.nk = K / kPipeK;
     if (const char *e = std::getenv("KR_GEMM_SK_WGS")) {
+        if (M < 256 || N < 256) return false;
         pl.G = std::max(1, std::atoi(e));
         if (pl.tiles >= pl.G || int64_t(pl.tiles) * pl.nk < 4 * int64_t(pl.G)) return false;
     } else {
-        const GemmTile dp = GemmPickTile(M, N, 0, false);
-        const int dp_tiles = ((M + dp.bm - 1) / dp.bm) * ((N + dp.bn - 1) / dp.bn);
-        const int dp_slots = CuCount() * (dp.bm * dp.bn >= 256 * 128 ? 1 : 2);
-        const int dp_rounds = (dp_tiles + dp_slots - 1) / dp_slots;
-        const double fill = double(dp_tiles) / (double(dp_rounds) * dp_slots);
-        static const bool longk = [] {
-            const char *e = std::getenv("KR_GEMM_SK_LONGK");
-            return e == nullptr || std::atoi(e) != 0;
-        }();
-        static const int longk_nk = [] {
-            const char *e = std::getenv("KR_GEMM_SK_LONGK_NK");
-            return e != nullptr ? std::max(32, std::atoi(e)) : 256;
-        }();
-        if (fill >= 0.6 && !(longk && fill < 0.9 && pl.nk >= longk_nk)) return false;
-        const int S = std::min(CuCount() / pl.tiles, pl.nk / 16);
+        const int S = M < 256 || N < 256 ? 0 : Split256Pieces(M, N, pl.tiles, pl.nk);
+        StreamKPlan small;
+        if (PlanSplit(M, N, K, S, small)) {
+            if (small.pmax < 2) return false;  // best as one piece per tile: data-parallel
+            pl = small;
+            return true;
+        }
         if (S < 2) return false;
         pl.G = S * pl.tiles;
     }
@@ -1151,6 +1302,28 @@ bool PlanStreamK(int M, int N, int K, StreamKPlan &pl)
     for (int t = 0; t < pl.tiles; ++t)
         pl.pmax = std::max(pl.pmax, owner(int64_t(t) * pl.nk + pl.nk - 1) - owner(int64_t(t) * pl.nk) + 1);
     return true;
+}
+
+// A split launch can release any relay tiles of whole 64-row blocks: a
+// finisher arrives on every relay tile its rows touch (ArriveRows), whether
+// they are whole row blocks or not.
+bool SplitPubOk(int M, int R) { return R > 0 && R % 64 == 0 && M % R == 0; }
+
+template <int DT, int BM, int BN>
+void LaunchSplit(const GemmParams &base, const StreamKPlan &pl, hipStream_t stream)
+{
+    GemmParams p = base;
+    p.tiles_m = (p.M + BM - 1) / BM;
+    p.tiles_n = (p.N + BN - 1) / BN;
+    if (p.tiles_m * p.tiles_n != pl.tiles || pl.G != pl.tiles * pl.pmax || pl.G > CuCount())
+        throw std::logic_error("gemm: split plan mismatch");
+    p.order_rows = 0;
+    p.group_m = RasterGroupM();
+    p.sk_wgs = pl.G;
+    p.sk_pmax = pl.pmax;
+    p.gemm_wgs = pl.G;
+    hipLaunchKernelGGL((GemmSplitKernel<DT, BM, BN, DeepStages<BM, BN>()>), dim3(pl.G), dim3(kThreads), 0, stream, p);
+    Check(hipGetLastError(), "gemm split launch");
 }
 
 template <int DT, int BM, int BN>
@@ -1164,13 +1337,10 @@ void LaunchTyped(const GemmParams &base, int order_rows, int tail_tiles, hipStre
     auto whole = [&](int rows) { return rows > 0 && rows % BM == 0 && p.tiles_m % (rows / BM) == 0; };
     p.order_rows = 0;
     if (p.pub.ctrl != nullptr && sk != nullptr) {
-        // stream-K: each tile's finisher arrives once on every relay tile its
-        // rows cover, so a relay tile waits for (row blocks in it) x tiles_n
-        // arrivals, or tiles_n when it is shorter than a row block
-        const int R = p.pub.rows_per_tile;
-        if (R <= 0 || (R % BM != 0 && BM % R != 0) || p.M % R != 0)
-            throw std::runtime_error("gemm: stream-K relay tiles must be whole row blocks or divide one");
-        p.pub.arrivals = (R >= BM ? R / BM : 1) * p.tiles_n;
+        // stream-K: each tile's finisher arrives on every relay tile its rows
+        // touch (ArriveRows counts the arrivals)
+        if (!SplitPubOk(p.M, p.pub.rows_per_tile))
+            throw std::runtime_error("gemm: stream-K relay tiles must be whole 64-row blocks dividing M");
     } else if (p.pub.ctrl != nullptr) {
         if (!whole(p.pub.rows_per_tile)) throw std::runtime_error("relay tile rows must be a multiple of BM dividing M");
         p.pub.arrivals = (p.pub.rows_per_tile / BM) * p.tiles_n;
@@ -1194,7 +1364,7 @@ void LaunchTyped(const GemmParams &base, int order_rows, int tail_tiles, hipStre
         // a grid resident as a whole releases every tile at about the same
         // time whatever the order: keep the grouped raster (square patches
         // per XCD, less operand traffic than relay-tile order)
-        if (sk == nullptr && p.gemm_wgs <= CuCount() * GemmWgsPerCu<DT, BM, BN>(p.K, false)) p.order_rows = 0;
+        if (sk == nullptr && p.gemm_wgs <= CuCount() * GemmWgsPerCu<DT, BM, BN>(p.M, p.N, p.K, false)) p.order_rows = 0;
     }
     if (sk != nullptr) {
         if (BM != 256 || BN != 256 || sk->tiles != p.gemm_wgs) throw std::logic_error("gemm: stream-K plan mismatch");
@@ -1209,7 +1379,7 @@ void LaunchTyped(const GemmParams &base, int order_rows, int tail_tiles, hipStre
     }
     const dim3 grid(grid_x);
     int threads = 0;
-    const GemmFn fn = PickGemmKernel<DT, BM, BN>(p.K, sk != nullptr, threads);
+    const GemmFn fn = PickGemmKernel<DT, BM, BN>(p.M, p.N, p.K, sk != nullptr, threads);
     void *args[] = {&p};
     Check(hipLaunchKernel(reinterpret_cast<const void *>(fn), grid, dim3(threads), args, 0, stream), "gemm launch");
 }
@@ -1218,66 +1388,93 @@ void LaunchTyped(const GemmParams &base, int order_rows, int tail_tiles, hipStre
 
 namespace {
 
-int Waves(int tiles, int slots) { return (tiles + slots - 1) / slots; }
+// Cheaper of 128 and 64 row tiles, one workgroup per CU on the deep ring
+// (bm -1: neither fits, or K keeps them off it).
+GemmTile PickSmallTile(int M, int N, int K, int relay_rows)
+{
+    GemmTile best{-1, -1};
+    double us = 1e30;
+    for (int bm : {128, 64}) {
+        const double t = relay_rows % bm == 0 ? SmallTileUs(bm, 1, M, N, K) : -1.0;
+        if (t < 0.0 || t >= us) continue;
+        us = t;
+        best = {bm, 128};
+    }
+    return best;
+}
+
+// Estimated time (us) of whole rounds of one of the larger tiles over K: its
+// time per 64-deep stage with the device full, one more per tile for its
+// prologue and epilogue, 6 for the launch. Fitted to rounds of 56..64 stages
+// (M 515..4096, N 4608..37888) and of 14; only the order of the candidates
+// matters, and where rounds are many and full the card's power limit levels
+// them (2048x37888x3584: 442..453 us whatever the tile).
+struct TileCost {
+    GemmTile tile;
+    int per_cu;
+    double stage;
+};
+constexpr TileCost kTileCosts[] = {
+    {{256, 256}, 1, 1.25}, {{192, 256}, 1, 1.05}, {{256, 128}, 1, 0.72}, {{128, 256}, 1, 0.73}, {{128, 128}, 2, 1.02}};
+
+double TileUs(const TileCost &c, int M, int N, int K)
+{
+    const int64_t tiles = int64_t((M + c.tile.bm - 1) / c.tile.bm) * ((N + c.tile.bn - 1) / c.tile.bn);
+    const int64_t slots = int64_t(CuCount()) * c.per_cu;
+    return 6.0 + double((tiles + slots - 1) / slots) * (K / kPipeK * c.stage + 1.0);
+}
 
 }  // namespace
 
-GemmTile GemmPickTile(int M, int N, int relay_rows, bool coresident)
+GemmTile GemmPickTile(int M, int N, int relay_rows, bool coresident, int K)
 {
-    // Candidates from most to least data reuse; take the first that keeps the
-    // device busy (>= 2 full waves of workgroups, or whole waves) or, failing
-    // that, the one with the best wave efficiency. A GEMM whose 128x128 tiles
-    // give every workgroup a CU of its own takes them: with so few workgroups
-    // each CU's load path is the limit, and smaller tiles put more CUs to work
-    // (MI355X, K 896: 2048x896 21.0 us against 24.0 for 128x256, 2048x1152
-    // 20.6 against 23.8). Every tile runs the same MFMA and K order, so the
-    // choice never changes the arithmetic.
-    static const GemmTile cands[] = {{256, 256}, {256, 128}, {128, 256}, {128, 128}, {64, 256}};
-    const int cus = 256;
-    if ((relay_rows == 0 || relay_rows % 128 == 0) && ((M + 127) / 128) * ((N + 127) / 128) <= cus)
-        return {128, 128};
-    // share of the device's slots the tiles' useful work fills
-    auto fill = [&](GemmTile t) {
-        const int tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-        const int slots = cus * (t.bm * t.bn >= 256 * 128 ? 1 : 2);
-        return double(M) * N / (double(Waves(tiles, slots)) * slots * t.bm * t.bn);
-    };
-    // 192x256 (three 32-row blocks per wave of the 8-wave grid) for a GEMM
-    // that 256x256 tiles leave a third idle and no smaller tile fills better,
-    // e.g. q/k/v 2048x4608: 198 tiles fill 75% against 144 tiles' 56%
-    // (without relay releases, waits or co-residency)
-    const bool try192 = relay_rows == 0 && !coresident;
-    GemmTile best{-1, -1};
-    double best_eff = -1.0;
-    auto pick192 = [&](GemmTile other) {
-        return try192 && fill({192, 256}) > 1.15 * fill(other) ? GemmTile{192, 256} : other;
-    };
-    for (const GemmTile &t : cands) {
-        if (relay_rows > 0 && relay_rows % t.bm != 0) continue;
-        if (coresident && t.bm * t.bn >= 256 * 256) continue;
-        const int tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-        const int slots = cus * (t.bm * t.bn >= 256 * 128 ? 1 : 2);
-        // enough workgroups for two rounds, or whole rounds exactly
-        if (tiles >= 2 * slots || tiles % slots == 0) return t.bm == 256 && t.bn == 256 ? t : pick192(t);
-        const double work = double(t.bm) * t.bn;  // per-workgroup work unit
-        const double eff = double(tiles) * work / (double(Waves(tiles, slots)) * slots * work);
-        const double score = eff * (t.bm * t.bn >= 256 * 128 ? 1.0 : 0.85);
-        if (score > best_eff) {
-            best_eff = score;
-            best = t;
+    // No relay and K on the pipelined kernels: the cheapest by the estimates
+    // above. Every tile runs the same MFMA and K order, so the choice never
+    // changes the arithmetic. Measured against the rule below, which knows
+    // neither K nor the tiles' rates: 515x24576x4096 177 -> 124 us,
+    // 1500x24576x4096 299 -> 253, 3072x6144x4096 173 -> 152, 3072x9728x896
+    // 79 -> 62, 2048x9728x896 59 -> 50.
+    const GemmTile small = PickSmallTile(M, N, K, relay_rows);
+    if (relay_rows == 0 && !coresident && K % kPipeK == 0 && !ForceSimple() && MainLoopMode() == 2) {
+        GemmTile best = small;
+        double us = small.bm > 0 ? SmallTileUs(small.bm, 1, M, N, K) : 1e30;
+        for (const TileCost &c : kTileCosts) {
+            const double t = TileUs(c, M, N, K);
+            if (t >= us) continue;
+            us = t;
+            best = c.tile;
         }
+        return best;
     }
-    return best.bm < 0 ? best : pick192(best);
+    if (small.bm > 0) return small;
+    return PickRelayTile(M, N, relay_rows, coresident);
+}
+
+// A small product whose cheapest row tile does not divide the relay tile (192
+// or 576 rows in 128 row tiles): GemmSplitKernel in one piece, which releases
+// any whole 64-row blocks (576x4096x4096, 64x256 tiles 61 us before).
+bool OnePieceRelay(int M, int N, int K, int relay_rows, StreamKPlan &pl)
+{
+    if (relay_rows <= 0 || !SplitPubOk(M, relay_rows) || ForceSimple() || MainLoopMode() != 2) return false;
+    const GemmTile t = PickSmallTile(M, N, K, 0);
+    if (t.bm < 0 || relay_rows % t.bm == 0) return false;
+    pl = StreamKPlan{};
+    pl.bm = t.bm;
+    pl.bn = t.bn;
+    pl.nk = K / kPipeK;
+    pl.tiles = pl.G = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    pl.pmax = 1;
+    return true;
 }
 
 bool GemmNormRelayFits(int M, int N, int K, int rows_per_tile, bool streamk_ws, int dtype)
 {
     if (AddRmsNormRowCpl(N) == 0 || rows_per_tile <= 0 || M % rows_per_tile != 0) return false;
     StreamKPlan skp;
-    const bool sk_pub_ok = rows_per_tile % 256 == 0 || 256 % rows_per_tile == 0;
-    if (streamk_ws && sk_pub_ok && !ForceSimple() && PlanStreamK(M, N, K, skp))
-        return NormRelayResident(dtype, 256, 256, M, N, K, rows_per_tile, skp.G);
-    GemmTile t = GemmPickTile(M, N, rows_per_tile, false);
+    if (streamk_ws && !ForceSimple() && PlanStreamK(M, N, K, skp) && SplitPubOk(M, rows_per_tile))
+        return NormRelayResident(dtype, skp.bm, skp.bn, M, N, K, rows_per_tile, skp.G);
+    if (OnePieceRelay(M, N, K, rows_per_tile, skp) && std::getenv("KR_GEMM_TILE") == nullptr) return true;
+    GemmTile t = GemmPickTile(M, N, rows_per_tile, false, K);
     if (const char *e = std::getenv("KR_GEMM_TILE")) {
         int bm = 0, bn = 0;
         if (std::sscanf(e, "%dx%d", &bm, &bn) == 2 && rows_per_tile % bm == 0) t = {bm, bn};
@@ -1290,7 +1487,7 @@ void GemmStreamKNeeds(int M, int N, int K, size_t *ws_bytes, int *counters)
 {
     StreamKPlan pl;
     if (PlanStreamK(M, N, K, pl)) {
-        *ws_bytes = size_t(pl.tiles) * pl.pmax * 256 * 256 * 4;
+        *ws_bytes = pl.WsBytes();
         *counters = pl.tiles;
     } else {
         *ws_bytes = 0;
@@ -1319,8 +1516,6 @@ bool SplitWaveTail(const GemmDesc &d, GemmDesc &a, GemmDesc &b)
         d.rope_cos != nullptr || d.norm_y != nullptr)
         return false;
     if (d.K % kPipeK != 0 || ForceSimple() || MainLoopMode() != 2 || PipeWaves() != 8) return false;
-    const GemmTile t = GemmPickTile(d.M, d.N, 0, false);
-    if (t.bm != 256 || t.bn != 256) return false;
     StreamKPlan skp;
     if (d.streamk && PlanStreamK(d.M, d.N, d.K, skp)) return false;
     const int64_t cus = CuCount();
@@ -1330,6 +1525,11 @@ bool SplitWaveTail(const GemmDesc &d, GemmDesc &a, GemmDesc &b)
     const int64_t n1 = rounds * cus / tm * 256;  // columns of the whole rounds
     const int64_t n2 = d.N - n1;
     if (n2 <= 0 || ((d.M + 191) / 192) * ((n2 + 255) / 256) > cus) return false;
+    // against the cheapest single launch (the second launch runs as the first
+    // drains: no launch time of its own)
+    double us = 1e30;
+    for (const TileCost &c : kTileCosts) us = std::min(us, TileUs(c, d.M, d.N, d.K));
+    if (TileUs(kTileCosts[0], d.M, int(n1), d.K) + TileUs(kTileCosts[1], d.M, int(n2), d.K) - 6.0 >= us) return false;
     a = d;
     b = d;
     a.N = int(n1);
@@ -1446,7 +1646,7 @@ void GemmLaunch(const GemmDesc &d, hipStream_t stream)
     }
     if (p.wait.ctrl != nullptr && p.wait.prod_rows <= 0) throw std::runtime_error("gemm: wait.prod_rows must be > 0");
     const int relay_rows = d.pub.ctrl != nullptr ? d.pub.rows_per_tile : 0;
-    GemmTile t = GemmPickTile(d.M, d.N, relay_rows, d.coresident);
+    GemmTile t = GemmPickTile(d.M, d.N, relay_rows, d.coresident, d.K);
     if (const char *e = std::getenv("KR_GEMM_TILE")) {
         // tile sweep override "BMxBN" (measurement aid; bits are unchanged)
         int bm = 0, bn = 0;
@@ -1460,7 +1660,6 @@ void GemmLaunch(const GemmDesc &d, hipStream_t stream)
         t.bn = d.bn;
     }
     if (t.bm < 0) throw std::runtime_error("gemm: relay tile rows must be a multiple of 64");
-    if (d.epi_act != nullptr && t.bn < 256) t = {t.bm >= 256 ? 256 : 128, 256};  // the epilogue pairs 16-col groups
     // 192x256 runs only on the staged 8-wave kernel; elsewhere 256x256 (the
     // same MFMA and K order: the same bits)
     if (t.bm == 192 && (d.K % kPipeK != 0 || ForceSimple() || MainLoopMode() != 2 ||
@@ -1475,18 +1674,32 @@ void GemmLaunch(const GemmDesc &d, hipStream_t stream)
         tail = d.tail_tiles > 0 ? std::min(d.tail_tiles, k) : k;
     }
     StreamKPlan skp;
-    // (a publishing split needs relay tiles that are whole 256-row blocks or
-    // divide one)
     const int rpt = d.pub.rows_per_tile;
-    const bool sk_pub_ok =
-        d.pub.ctrl == nullptr || (rpt > 0 && (rpt % 256 == 0 || 256 % rpt == 0) && d.M % rpt == 0);
-    if (d.streamk && sk_pub_ok && d.wait.ctrl == nullptr && d.tail_act == nullptr && d.epi_act == nullptr && !ForceSimple() &&
-        d.bm == 0 && d.bn == 0 && PlanStreamK(d.M, d.N, d.K, skp) && d.sk_ws != nullptr && d.sk_cnt != nullptr &&
-        d.sk_ws_bytes >= size_t(skp.tiles) * skp.pmax * 256 * 256 * 4 && d.sk_cnt_len >= skp.tiles &&
+    if (d.streamk && d.wait.ctrl == nullptr && d.tail_act == nullptr && d.epi_act == nullptr && !ForceSimple() &&
+        d.bm == 0 && d.bn == 0 && PlanStreamK(d.M, d.N, d.K, skp) &&
+        (d.pub.ctrl == nullptr || SplitPubOk(d.M, rpt)) && d.sk_ws != nullptr && d.sk_cnt != nullptr &&
+        d.sk_ws_bytes >= skp.WsBytes() && d.sk_cnt_len >= skp.tiles &&
         (d.norm_y == nullptr || skp.G <= CuCount())) {
         p.sk_ws = static_cast<float *>(d.sk_ws);
         p.sk_cnt = d.sk_cnt;
+        if (skp.bm == 128) {
+            bf ? LaunchSplit<kBF16, 128, 128>(p, skp, stream) : LaunchSplit<kF16, 128, 128>(p, skp, stream);
+            return;
+        }
+        if (skp.bm == 64) {
+            bf ? LaunchSplit<kBF16, 64, 128>(p, skp, stream) : LaunchSplit<kF16, 64, 128>(p, skp, stream);
+            return;
+        }
         bf ? LaunchTyped<kBF16, 256, 256>(p, 0, 0, stream, &skp) : LaunchTyped<kF16, 256, 256>(p, 0, 0, stream, &skp);
+        return;
+    }
+    if (OnePieceRelay(d.M, d.N, d.K, relay_rows, skp) && d.bm == 0 && d.bn == 0 && std::getenv("KR_GEMM_TILE") == nullptr &&
+        d.wait.ctrl == nullptr && d.tail_act == nullptr && d.epi_act == nullptr && d.order_rows == 0) {
+        if (skp.bm == 128) {
+            bf ? LaunchSplit<kBF16, 128, 128>(p, skp, stream) : LaunchSplit<kF16, 128, 128>(p, skp, stream);
+        } else {
+            bf ? LaunchSplit<kBF16, 64, 128>(p, skp, stream) : LaunchSplit<kF16, 64, 128>(p, skp, stream);
+        }
         return;
     }
 #define KR_GEMM_CASE(BM_, BN_)                                                                     \
@@ -1500,6 +1713,7 @@ void GemmLaunch(const GemmDesc &d, hipStream_t stream)
     KR_GEMM_CASE(256, 128)
     KR_GEMM_CASE(128, 256)
     KR_GEMM_CASE(128, 128)
+    KR_GEMM_CASE(64, 128)
     KR_GEMM_CASE(64, 256)
 #undef KR_GEMM_CASE
     throw std::runtime_error("gemm: unsupported tile " + std::to_string(t.bm) + "x" + std::to_string(t.bn));

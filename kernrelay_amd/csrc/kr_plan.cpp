@@ -720,7 +720,7 @@ private:
         if (EnvInt("KR_PLAN_CORESIDENT", 0) != 0) return true;
         const int64_t prows = L.pub_rows > 0 ? L.pub_rows : TaskRows(*L.task);
         const int N = int(L.task->n_tile > 0 ? L.task->n_tile : L.node->n);
-        const GemmTile best = GemmPickTile(int(TaskRows(*L.task)), N, int(prows), false);
+        const GemmTile best = GemmPickTile(int(TaskRows(*L.task)), N, int(prows), false, int(L.node->k));
         return !(best.bm == 256 && best.bn == 256);
     }
 
@@ -787,7 +787,7 @@ private:
         const int64_t prows = PL.pub_rows;
         if (prows <= 0 || L.tile_rows != prows || in_off % prows != 0) return -1;
         const int M = int(TaskRows(*PL.task)), N = int(P.n);
-        const GemmTile gt = GemmPickTile(M, N, int(prows), PL.coresident);
+        const GemmTile gt = GemmPickTile(M, N, int(prows), PL.coresident, int(P.k));
         if (gt.bm <= 0) return -1;
         const int64_t tn = (N + gt.bn - 1) / gt.bn;
         const int64_t per = (prows / gt.bm) * tn;                 // workgroups per relay tile
@@ -1169,7 +1169,7 @@ private:
                 d.y_dtype = c.out_dtype;
                 d.ld_y = c.cols;
             }
-            if (pub.ctrl && GemmPickTile(d.M, d.N, pub.rows_per_tile, d.coresident).bm < 0) {
+            if (pub.ctrl && GemmPickTile(d.M, d.N, pub.rows_per_tile, d.coresident, d.K).bm < 0) {
                 // the tile cannot be one GEMM relay tile: release after the GEMM
                 GemmLaunch(d, s);
                 for (int k = 0; k < L.merged; ++k) PublishLaunch(pub, k, s);
