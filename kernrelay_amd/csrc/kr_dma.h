@@ -32,6 +32,14 @@ __device__ __forceinline__ void DmaLoad16(const void *gptr, uint32_t lds_addr)
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(lds_addr) : "memory");
 }
 
+// The same with the lanes' addresses as a wave-uniform base plus a 32-bit
+// byte offset each (scalar address arithmetic, one register per lane).
+__device__ __forceinline__ void DmaLoad16S(const void *base, uint32_t off, uint32_t lds_addr)
+{
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_addr)
+                 : "memory");
+}
+
 __device__ __forceinline__ void DmaTouch4(const void *gptr, uint32_t lds_addr)
 {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(gptr), "s"(lds_addr) : "memory");

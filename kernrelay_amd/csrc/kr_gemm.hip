@@ -1043,6 +1043,25 @@ bool DeepGrid(int bm, int bn, int M, int N)
     return ((M + bm - 1) / bm) * ((N + bn - 1) / bn) <= CuCount();
 }
 
+// Whether the launch's 256-wide tiles run the wide loop: K of at least 32
+// stages (its 4-wave prologue and epilogue, one wave per SIMD, cost more than
+// the 8-wave kernel's: 16384x2048x1024 71 -> 74 us), and workgroups for three
+// quarters of the CUs (with fewer the other loops were as fast or faster:
+// 2048x3584x3584 in 256x256 tiles 79 against 82 us, 1024x3584x3584 in
+// 256x128 48.6 against 49.6; full: 8192^3 789 -> 750, 4096x24576x4096 629 ->
+// 611, 2048x4096x12288 in 256x128 tiles 176 -> 163).
+// Its tile rows are addressed by 32-bit byte offsets: `stride` (elements) must
+// keep 256 of them below 4 GB.
+bool WideLoop(int bm, int bn, int M, int N, int K, int64_t stride)
+{
+    if (stride >= (int64_t(1) << 23)) return false;
+    if (K % kPipeK != 0 || K < 32 * kPipeK || ForceSimple() || MainLoopMode() != 2 || PipeWaves() != 8 ||
+        PrefetchStages() != 0)
+        return false;
+    if (bm * bn != 256 * 128 && bm * bn != 256 * 256) return false;
+    return int64_t((M + bm - 1) / bm) * ((N + bn - 1) / bn) * 4 >= int64_t(CuCount()) * 3;
+}
+
 using GemmFn = void (*)(GemmParams);
 
 // The kernel a launch of BM x BN tiles runs over K, and its block size: the
@@ -1050,9 +1069,9 @@ using GemmFn = void (*)(GemmParams);
 // or data-parallel) unless KR_GEMM_WAVES=4; the 4-wave pipelined kernel for
 // the other tiles; the simple kernel where K % 64 != 0 or KR_GEMM_SIMPLE=1.
 // A small tile whose grid has at most one workgroup per CU takes the deep
-// ring.
+// ring; 256-wide tiles with K long enough the wide loop.
 template <int DT, int BM, int BN>
-GemmFn PickGemmKernel(int M, int N, int K, bool sk, int &threads)
+GemmFn PickGemmKernel(int M, int N, int K, int64_t stride, bool sk, int &threads)
 {
     if constexpr (BM == 192) {
         // 192x256: the 8-wave staged kernel only (GemmLaunch picks this tile
@@ -1064,6 +1083,12 @@ GemmFn PickGemmKernel(int M, int N, int K, bool sk, int &threads)
         return GemmPipeKernel<DT, BM, BN, 0, 8, false, 2>;
     } else {
         if (K % kPipeK == 0 && !ForceSimple()) {
+            if constexpr (BM * BN >= 128 * 256) {
+                if (WideLoop(BM, BN, M, N, K, stride) && !sk) {
+                    threads = kThreads;
+                    return GemmPipeKernel<DT, BM, BN, 0, 4, false, 3>;
+                }
+            }
             if constexpr (BM == 256 && BN == 256) {
                 if (sk) {
                     threads = 512;
@@ -1093,15 +1118,15 @@ GemmFn PickGemmKernel(int M, int N, int K, bool sk, int &threads)
 
 // Workgroups of that kernel one CU holds at once, from the runtime's
 // occupancy query on the exact instantiation (registers, LDS, waves);
-// cached per (dtype, tile, K-path, stream-K, ring).
+// cached per (dtype, tile, K-path, stream-K, ring, loop).
 template <int DT, int BM, int BN>
-int GemmWgsPerCu(int M, int N, int K, bool sk)
+int GemmWgsPerCu(int M, int N, int K, int64_t stride, bool sk)
 {
-    static int cache[2][2][2] = {};  // 0: not asked yet
-    int &c = cache[K % kPipeK == 0][sk][DeepGrid(BM, BN, M, N)];
+    static int cache[2][2][2][2] = {};  // 0: not asked yet
+    int &c = cache[K % kPipeK == 0][sk][DeepGrid(BM, BN, M, N)][WideLoop(BM, BN, M, N, K, stride)];
     if (c == 0) {
         int threads = 0;
-        const GemmFn fn = PickGemmKernel<DT, BM, BN>(M, N, K, sk, threads);
+        const GemmFn fn = PickGemmKernel<DT, BM, BN>(M, N, K, stride, sk, threads);
         int n = 0;
         Check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void *>(fn), threads, 0),
               "gemm occupancy");
@@ -1111,11 +1136,12 @@ int GemmWgsPerCu(int M, int N, int K, bool sk)
     return c;
 }
 
-int GemmWgsPerCu(int dt, int bm, int bn, int M, int N, int K, bool sk)
+int GemmWgsPerCu(int dt, int bm, int bn, int M, int N, int K, int64_t stride, bool sk)
 {
     const bool bf = dt == kBF16;
 #define KR_OCC_CASE(BM_, BN_) \
-    if (bm == BM_ && bn == BN_) return bf ? GemmWgsPerCu<kBF16, BM_, BN_>(M, N, K, sk) : GemmWgsPerCu<kF16, BM_, BN_>(M, N, K, sk);
+    if (bm == BM_ && bn == BN_) return bf ? GemmWgsPerCu<kBF16, BM_, BN_>(M, N, K, stride, sk) \
+                                                  : GemmWgsPerCu<kF16, BM_, BN_>(M, N, K, stride, sk);
     KR_OCC_CASE(256, 256)
     KR_OCC_CASE(192, 256)
     KR_OCC_CASE(256, 128)
@@ -1137,10 +1163,10 @@ int GemmWgsPerCu(int dt, int bm, int bn, int M, int N, int K, bool sk)
 bool NormRelayResident(int dt, int bm, int bn, int M, int N, int K, int rows_per_tile, int sk_wgs)
 {
     if (sk_wgs > 0 && bm < 256) return sk_wgs <= CuCount();  // GemmSplitKernel: one per CU
-    if (sk_wgs > 0) return sk_wgs <= CuCount() * GemmWgsPerCu(dt, 256, 256, M, N, K, true);
+    if (sk_wgs > 0) return sk_wgs <= CuCount() * GemmWgsPerCu(dt, 256, 256, M, N, K, K, true);
     if (rows_per_tile <= 0 || rows_per_tile % bm != 0 || M % rows_per_tile != 0) return false;
     const int per = (rows_per_tile / bm) * ((N + bn - 1) / bn);
-    return per <= CuCount() * GemmWgsPerCu(dt, bm, bn, M, N, K, false);
+    return per <= CuCount() * GemmWgsPerCu(dt, bm, bn, M, N, K, K, false);
 }
 
 // Estimated time (us) of a 256x256 split in S pieces (the last one sums all
@@ -1364,7 +1390,7 @@ void LaunchTyped(const GemmParams &base, int order_rows, int tail_tiles, hipStre
         // a grid resident as a whole releases every tile at about the same
         // time whatever the order: keep the grouped raster (square patches
         // per XCD, less operand traffic than relay-tile order)
-        if (sk == nullptr && p.gemm_wgs <= CuCount() * GemmWgsPerCu<DT, BM, BN>(p.M, p.N, p.K, false)) p.order_rows = 0;
+        if (sk == nullptr && p.gemm_wgs <= CuCount() * GemmWgsPerCu<DT, BM, BN>(p.M, p.N, p.K, std::max(p.lda, p.ldb), false)) p.order_rows = 0;
     }
     if (sk != nullptr) {
         if (BM != 256 || BN != 256 || sk->tiles != p.gemm_wgs) throw std::logic_error("gemm: stream-K plan mismatch");
@@ -1379,7 +1405,7 @@ void LaunchTyped(const GemmParams &base, int order_rows, int tail_tiles, hipStre
     }
     const dim3 grid(grid_x);
     int threads = 0;
-    const GemmFn fn = PickGemmKernel<DT, BM, BN>(p.M, p.N, p.K, sk != nullptr, threads);
+    const GemmFn fn = PickGemmKernel<DT, BM, BN>(p.M, p.N, p.K, std::max(p.lda, p.ldb), sk != nullptr, threads);
     void *args[] = {&p};
     Check(hipLaunchKernel(reinterpret_cast<const void *>(fn), grid, dim3(threads), args, 0, stream), "gemm launch");
 }
