@@ -7,7 +7,9 @@
 #include <algorithm>
 #include <chrono>
 #include <cstdlib>
+#include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "kr_common.h"
@@ -117,6 +119,72 @@ inline std::vector<uint32_t> ReservedCuMask(int num_cus, int per_xcd)
     return mask;
 }
 
+// Idle CU-masked streams between runs. Making one (a hardware queue) takes 3.5
+// to 6 ms and destroying it 1.5 to 3, 14 ms for a run's pair: more than the
+// rest of a small schedule's run (1024x512x1024 with three consumers: 20 ms).
+// A stream in use belongs to its run alone (taken out of the pool); it comes
+// back idle, outside any capture, and at most kMaxIdle wait here, the oldest
+// giving way. A stream that reports an error, in either direction, is dropped.
+class QueueStreams {
+public:
+    static QueueStreams &Get()
+    {
+        static QueueStreams pool;
+        return pool;
+    }
+    // A stream of `device` (current) limited to the CUs of `mask`.
+    hipStream_t Take(int device, const std::vector<uint32_t> &mask, const char *what)
+    {
+        for (;;) {
+            hipStream_t s = nullptr;
+            {
+                std::lock_guard<std::mutex> lock(mu_);
+                auto it = std::find_if(idle_.begin(), idle_.end(),
+                                       [&](const Idle &i) { return i.device == device && i.mask == mask; });
+                if (it == idle_.end()) break;
+                s = it->stream;
+                idle_.erase(it);
+            }
+            // a device reset invalidates the handle: forget it
+            const hipError_t rc = hipStreamQuery(s);
+            if (rc == hipSuccess || rc == hipErrorNotReady) return s;
+            (void)hipGetLastError();
+        }
+        hipStream_t s = nullptr;
+        Check(hipExtStreamCreateWithCUMask(&s, uint32_t(mask.size()), mask.data()), what);
+        return s;
+    }
+    void Return(int device, std::vector<uint32_t> mask, hipStream_t s)
+    {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        bool ok = hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+        ok = ok && hipStreamSynchronize(s) == hipSuccess;
+        if (ok) {
+            std::lock_guard<std::mutex> lock(mu_);
+            idle_.push_back({device, std::move(mask), s});
+            if (idle_.size() <= kMaxIdle) return;
+            s = idle_.front().stream;
+            idle_.erase(idle_.begin());
+        }
+        (void)hipStreamDestroy(s);
+    }
+
+private:
+    struct Idle {
+        int device;
+        std::vector<uint32_t> mask;
+        hipStream_t stream;
+    };
+    static constexpr size_t kMaxIdle = 4;
+    QueueStreams() = default;
+    ~QueueStreams()
+    {
+        for (const Idle &i : idle_) (void)hipStreamDestroy(i.stream);
+    }
+    std::mutex mu_;
+    std::vector<Idle> idle_;
+};
+
 // Producer + consumer stream pair, each on its own hardware queue.
 //
 // The relay waits in both directions on the device, so the two streams must
@@ -138,30 +206,33 @@ struct StreamPair {
     hipStream_t cons = nullptr;
     int cons_cus = 0;  // CUs in the consumer mask
     int prod_cus = 0;
+    int device = 0;
+    std::vector<uint32_t> pmask, cmask;
 
-    void Create(int device, int partition_per_xcd = 0)
+    void Create(int dev, int partition_per_xcd = 0)
     {
+        device = dev;
         hipDeviceProp_t prop;
         Check(hipGetDeviceProperties(&prop, device), "device props");
         const int ncu = prop.multiProcessorCount;
         std::vector<uint32_t> all((ncu + 31) / 32, 0u);
         for (int c = 0; c < ncu; ++c) all[c / 32] |= 1u << (c % 32);
-        std::vector<uint32_t> pmask = all, cmask = all;
+        pmask = cmask = all;
         if (partition_per_xcd > 0) {
             cmask = ReservedCuMask(ncu, partition_per_xcd);
             for (size_t i = 0; i < pmask.size(); ++i) pmask[i] &= ~cmask[i];
         } else if (const int per_xcd = EnvInt("KR_CONSUMER_CUS_PER_XCD", 0); per_xcd > 0) {
             cmask = ReservedCuMask(ncu, std::min(per_xcd, 4));
         }
-        Check(hipExtStreamCreateWithCUMask(&prod, uint32_t(pmask.size()), pmask.data()), "create producer stream");
-        Check(hipExtStreamCreateWithCUMask(&cons, uint32_t(cmask.size()), cmask.data()), "create consumer stream");
+        prod = QueueStreams::Get().Take(device, pmask, "create producer stream");
+        cons = QueueStreams::Get().Take(device, cmask, "create consumer stream");
         for (uint32_t w : pmask) prod_cus += __builtin_popcount(w);
         for (uint32_t w : cmask) cons_cus += __builtin_popcount(w);
     }
     void Destroy()
     {
-        if (prod) (void)hipStreamDestroy(prod);
-        if (cons) (void)hipStreamDestroy(cons);
+        if (prod) QueueStreams::Get().Return(device, pmask, prod);
+        if (cons) QueueStreams::Get().Return(device, cmask, cons);
         prod = cons = nullptr;
     }
 };
