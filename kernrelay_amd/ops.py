@@ -77,15 +77,21 @@ def _lib():
     return L
 
 
+# A launch's host side is Python for the most part, and the small kernels run
+# in less time than it took (a gemm of a few rows: 5 us on the GPU, 8.5 per
+# call): dtypes come from one table, addresses go to ctypes as plain ints, and
+# the current stream's handle is read without making a torch Stream for it.
+_DT = {}
+
+
 def _dt(t):
-    import torch
-    if t.dtype == torch.bfloat16:
-        return KR_BF16
-    if t.dtype == torch.float16:
-        return KR_F16
-    if t.dtype == torch.float32:
-        return KR_F32
-    raise TypeError("unsupported dtype %s" % t.dtype)
+    if not _DT:
+        import torch
+        _DT.update({torch.bfloat16: KR_BF16, torch.float16: KR_F16, torch.float32: KR_F32})
+    try:
+        return _DT[t.dtype]
+    except KeyError:
+        raise TypeError("unsupported dtype %s" % t.dtype) from None
 
 
 def _ptr(t):
@@ -93,13 +99,25 @@ def _ptr(t):
         return None
     if not t.is_cuda:
         raise RuntimeError("kernrelay ops need device tensors (got a CPU tensor)")
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
+
+
+_RAW = None  # (current device, current stream handle of a device)
 
 
 def _stream(stream):
-    import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    if stream is not None:
+        return stream.cuda_stream
+    global _RAW
+    if _RAW is None:
+        import torch
+        torch.cuda.current_stream()  # initialises the device as any torch call does
+        get = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if get is None:  # a torch without the raw accessor
+            _RAW = (int, lambda _: torch.cuda.current_stream().cuda_stream)
+        else:
+            _RAW = (torch._C._cuda_getDevice, get)
+    return _RAW[1](_RAW[0]())
 
 
 class QueueStream:
