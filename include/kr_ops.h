@@ -138,10 +138,10 @@ int kr_op_gemm_add_rmsnorm(int dtype, const void *A, int64_t lda, const void *Bt
                            float eps, const kr_pub *pub, uint32_t max_spins, void *ws, size_t ws_bytes,
                            int32_t *counters, int n_counters, void *stream);
 
-/* Stream-K GEMM for shapes whose 256x256 output tiles are fewer than the CUs
+/* Split-K GEMM for shapes whose output tiles are fewer than the CUs
  * (the reference's q/k/v, o and down projections at prefill sizes,
- * exec/qwen_main.cpp:499-512, 1336-1344): every CU takes an equal run of the
- * (tile, K stage) iterations, and a tile split between CUs is summed in fixed
+ * exec/qwen_main.cpp:499-512, 1336-1344): each tile (256x256, or 64 / 128 x
+ * 128 below 1920 rows) runs in pieces of K on as many CUs, summed in fixed
  * piece order by the last of them, so the bits depend on the shape only (a
  * row-split launch of the same GEMM would differ; use it where no launch is
  * split). Same operands and rounding as kr_op_gemm (bias added to the

@@ -43,10 +43,10 @@ struct GemmDesc {
     int y_op = 0;
     int y_dtype = 0;
     int64_t ld_y = 0;
-    // Stream-K (no relay on this launch): when the 256x256 tiles are fewer
-    // than the CUs, every CU takes an equal share of the (tile, K stage)
-    // iterations and split tiles are summed in piece order by their last
-    // piece. Needs the caller's workspace (GemmStreamKNeeds); the counters
+    // Split K: a product whose tiles leave CUs idle runs each tile in pieces
+    // of K (256x256 tiles, or 64/128 x 128 ones below 1920 rows), summed in
+    // piece order by the last of them; with a release, relay tiles of whole
+    // 64-row blocks. Needs the caller's workspace (GemmStreamKNeeds); the counters
     // must be zero before the first launch and stay owned by one stream.
     // Bits depend on the shape only, so a launch that never runs row-split
     // is reproducible; silently data-parallel when the plan does not apply.

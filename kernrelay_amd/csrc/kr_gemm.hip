@@ -9,7 +9,8 @@
 //   256x256 tiles 8 waves in a 2x4 grid (128x64 each, two waves per SIMD), as
 //   32x32 accumulator blocks (fp32). The 8-wave register-staged kernels and
 //   the simple kernel compute a block as four 16x16 sub-blocks with
-//   v_mfma_f32_16x16x32 (4 values per lane each); the 4-wave direct-to-LDS
+//   v_mfma_f32_16x16x32 (4 values per lane each), and so does the 4-wave wide
+//   loop of the 256-wide tiles with long K; the other 4-wave direct-to-LDS
 //   kernels as one block with v_mfma_f32_32x32x16 (16 values per lane). The
 //   16x16x32 instruction reads and writes a quarter of the accumulator
 //   registers of 32x32x16 per flop; under the card's power limit an
