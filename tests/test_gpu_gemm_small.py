@@ -20,8 +20,9 @@ BF, HF = torch.bfloat16, torch.float16
 
 def make(M, N, K, dt, bias, seed):
     g = torch.Generator(device="cuda").manual_seed(seed)
-    x = torch.randn(M, K, device="cuda", generator=g).to(dt)
-    w = (torch.randn(N, K, device="cuda", generator=g) * 0.02).to(dt)
+    # views into wider buffers: row strides beyond K, different for x and w
+    x = torch.randn(M, K + 24, device="cuda", generator=g).to(dt)[:, :K]
+    w = (torch.randn(N, K + 8, device="cuda", generator=g) * 0.02).to(dt)[:, :K]
     b = (torch.randn(N, device="cuda", generator=g) * 0.5).to(dt) if bias else None
     return x, w, b
 
