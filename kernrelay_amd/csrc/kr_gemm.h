@@ -116,4 +116,16 @@ struct GemmTile {
 // choice without a relay depends on it).
 GemmTile GemmPickTile(int M, int N, int relay_rows, bool coresident = false, int K = 4096);
 
+// The main loops of the GEMM kernels (kr_gemm.hip, kr_gemm_pipe.inc).
+enum class GemmLoop { kSimple, kRing, kDeep, kStaged, kWide };
+
 }  // namespace kr
+
+// What GemmLaunch runs for a product of these sizes and row strides
+// (elements): its tile, its loop (kr::GemmLoop) and the pieces of K each tile
+// is cut into (1: whole). relay_rows > 0: it releases relay tiles of that many
+// rows; ws: the caller gives the workspace GemmStreamKNeeds asks for; norm: with
+// the Add+RMSNorm relay consumer. Launches nothing. Non-zero: it would be
+// refused.
+extern "C" int kr_gemm_route(int M, int N, int K, int64_t lda, int64_t ldb, int relay_rows, int ws, int norm, int *bm,
+                             int *bn, int *loop, int *pieces);

@@ -1063,17 +1063,28 @@ bool WideLoop(int bm, int bn, int M, int N, int K, int64_t stride)
     return int64_t((M + bm - 1) / bm) * ((N + bn - 1) / bn) * 4 >= int64_t(CuCount()) * 3;
 }
 
+// The loop a launch of bm x bn tiles runs over K: the simple kernel where
+// K % 64 != 0 or KR_GEMM_SIMPLE=1; the 8-wave kernel for 192x256 and 256x256
+// (stream-K or data-parallel) unless KR_GEMM_WAVES=4; the wide loop for
+// 256-wide tiles with K long enough; the deep ring for a small tile whose
+// grid has at most one workgroup per CU; the 4-wave ring for the others.
+GemmLoop LoopOf(int bm, int bn, int M, int N, int K, int64_t stride, bool sk)
+{
+    if (bm == 192) return GemmLoop::kStaged;
+    if (K % kPipeK != 0 || ForceSimple()) return GemmLoop::kSimple;
+    if (!sk && WideLoop(bm, bn, M, N, K, stride)) return GemmLoop::kWide;
+    if (bm == 256 && bn == 256 && (sk || PipeWaves() == 8)) return GemmLoop::kStaged;
+    if (bm * bn < 256 * 128 && bn == 128 && DeepGrid(bm, bn, M, N)) return GemmLoop::kDeep;
+    return GemmLoop::kRing;
+}
+
 using GemmFn = void (*)(GemmParams);
 
-// The kernel a launch of BM x BN tiles runs over K, and its block size: the
-// 8-wave staged kernel for 192x256; for 256x256 the 8-wave kernel (stream-K
-// or data-parallel) unless KR_GEMM_WAVES=4; the 4-wave pipelined kernel for
-// the other tiles; the simple kernel where K % 64 != 0 or KR_GEMM_SIMPLE=1.
-// A small tile whose grid has at most one workgroup per CU takes the deep
-// ring; 256-wide tiles with K long enough the wide loop.
+// The kernel of LoopOf's choice, and its block size.
 template <int DT, int BM, int BN>
 GemmFn PickGemmKernel(int M, int N, int K, int64_t stride, bool sk, int &threads)
 {
+    [[maybe_unused]] const GemmLoop loop = LoopOf(BM, BN, M, N, K, stride, sk);
     if constexpr (BM == 192) {
         // 192x256: the 8-wave staged kernel only (GemmLaunch picks this tile
         // only where that kernel runs)
@@ -1083,48 +1094,43 @@ GemmFn PickGemmKernel(int M, int N, int K, int64_t stride, bool sk, int &threads
         threads = 512;
         return GemmPipeKernel<DT, BM, BN, 0, 8, false, 2>;
     } else {
-        if (K % kPipeK == 0 && !ForceSimple()) {
-            if constexpr (BM * BN >= 128 * 256) {
-                if (WideLoop(BM, BN, M, N, K, stride) && !sk) {
-                    threads = kThreads;
-                    return GemmPipeKernel<DT, BM, BN, 0, 4, false, 3>;
-                }
+        if constexpr (BM * BN >= 128 * 256) {
+            if (loop == GemmLoop::kWide) {
+                threads = kThreads;
+                return GemmPipeKernel<DT, BM, BN, 0, 4, false, 3>;
             }
-            if constexpr (BM == 256 && BN == 256) {
-                if (sk) {
-                    threads = 512;
+        }
+        if constexpr (BM == 256 && BN == 256) {
+            if (loop == GemmLoop::kStaged) {
+                threads = 512;
+                if (sk)
                     return MainLoopMode() == 2 ? GemmPipeKernel<DT, BM, BN, 0, 8, true, 2>
                                                : GemmPipeKernel<DT, BM, BN, 0, 8, true>;
-                }
-                if (PipeWaves() == 8) {
-                    threads = 512;
-                    return MainLoopMode() == 2 ? GemmPipeKernel<DT, BM, BN, 0, 8, false, 2>
-                                               : GemmPipeKernel<DT, BM, BN, 0, 8>;
-                }
-            }
-            threads = kThreads;
-            if constexpr (BM * BN < 256 * 128 && BN == 128) {
-                if (DeepGrid(BM, BN, M, N)) return GemmPipeKernel<DT, BM, BN, 0, 4, false, 0, DeepStages<BM, BN>()>;
-            }
-            switch (PrefetchStages()) {
-            case 2: return GemmPipeKernel<DT, BM, BN, 2, 4>;
-            case 4: return GemmPipeKernel<DT, BM, BN, 4, 4>;
-            default: return GemmPipeKernel<DT, BM, BN, 0, 4>;
+                return MainLoopMode() == 2 ? GemmPipeKernel<DT, BM, BN, 0, 8, false, 2>
+                                           : GemmPipeKernel<DT, BM, BN, 0, 8>;
             }
         }
         threads = kThreads;
-        return GemmKernel<DT, BM, BN>;
+        if (loop == GemmLoop::kSimple) return GemmKernel<DT, BM, BN>;
+        if constexpr (BM * BN < 256 * 128 && BN == 128) {
+            if (loop == GemmLoop::kDeep) return GemmPipeKernel<DT, BM, BN, 0, 4, false, 0, DeepStages<BM, BN>()>;
+        }
+        switch (PrefetchStages()) {
+        case 2: return GemmPipeKernel<DT, BM, BN, 2, 4>;
+        case 4: return GemmPipeKernel<DT, BM, BN, 4, 4>;
+        default: return GemmPipeKernel<DT, BM, BN, 0, 4>;
+        }
     }
 }
 
 // Workgroups of that kernel one CU holds at once, from the runtime's
 // occupancy query on the exact instantiation (registers, LDS, waves);
-// cached per (dtype, tile, K-path, stream-K, ring, loop).
+// cached per (dtype, tile, stream-K, loop).
 template <int DT, int BM, int BN>
 int GemmWgsPerCu(int M, int N, int K, int64_t stride, bool sk)
 {
-    static int cache[2][2][2][2] = {};  // 0: not asked yet
-    int &c = cache[K % kPipeK == 0][sk][DeepGrid(BM, BN, M, N)][WideLoop(BM, BN, M, N, K, stride)];
+    static int cache[2][5] = {};  // 0: not asked yet
+    int &c = cache[sk][int(LoopOf(BM, BN, M, N, K, stride, sk))];
     if (c == 0) {
         int threads = 0;
         const GemmFn fn = PickGemmKernel<DT, BM, BN>(M, N, K, stride, sk, threads);
@@ -1178,14 +1184,15 @@ double Split256Us(int K, int S)
 }
 
 // Estimated time (us) of a product in bm x 128 tiles, one workgroup per CU on
-// the deep ring, each tile in S pieces of K; negative when that does not fit.
+// the deep ring, each tile in S pieces of K (two stages or more in each);
+// negative when that does not fit.
 // Fitted to M 37..1500 at the projections of the three shipped models (within
 // 15%): a launch costs 6, a stage 0.24 (64 rows) / 0.32 (128) alone and 0.38 /
 // 0.59 with every CU loading, a fix-up 2 plus 0.5 / 1.4 a piece.
 double SmallTileUs(int bm, int S, int M, int N, int K)
 {
     const int tiles = ((M + bm - 1) / bm) * ((N + 127) / 128), G = tiles * S, nk = K / kPipeK;
-    if (K % kPipeK != 0 || G > CuCount() || nk < 2 * S) return -1.0;
+    if (K % kPipeK != 0 || G > CuCount() || (S > 1 && nk < 2 * S)) return -1.0;
     const double load = double(G) / CuCount();
     const double stage = bm == 64 ? 0.24 + 0.14 * load : 0.32 + 0.27 * load;
     const double fix = S > 1 ? 2.0 + (bm == 64 ? 0.5 : 1.4) * S : 0.0;
@@ -1572,6 +1579,53 @@ bool SplitWaveTail(const GemmDesc &d, GemmDesc &a, GemmDesc &b)
     return true;
 }
 
+namespace {
+
+// What a launch runs: a split plan (G > 0), or data-parallel tiles t.
+struct Route {
+    StreamKPlan split;
+    GemmTile t{-1, -1};
+};
+
+Route RouteOf(const GemmDesc &d)
+{
+    const int relay_rows = d.pub.ctrl != nullptr ? d.pub.rows_per_tile : 0;
+    GemmTile t = GemmPickTile(d.M, d.N, relay_rows, d.coresident, d.K);
+    const char *forced = std::getenv("KR_GEMM_TILE");
+    if (forced != nullptr) {
+        // tile sweep override "BMxBN" (measurement aid; bits are unchanged)
+        int bm = 0, bn = 0;
+        if (std::sscanf(forced, "%dx%d", &bm, &bn) == 2 && (relay_rows == 0 || relay_rows % bm == 0)) t = {bm, bn};
+    }
+    if (d.bm > 0) {
+        // a forced M tile pairs with the widest N tile built for it
+        t.bm = d.bm;
+        t.bn = d.bn > 0 ? d.bn : 256;
+    } else if (d.bn > 0) {
+        t.bn = d.bn;
+    }
+    if (t.bm < 0) throw std::runtime_error("gemm: relay tile rows must be a multiple of 64");
+    // 192x256 runs only on the staged 8-wave kernel; elsewhere 256x256 (the
+    // same MFMA and K order: the same bits)
+    if (t.bm == 192 && (d.K % kPipeK != 0 || ForceSimple() || MainLoopMode() != 2 ||
+                        d.tail_act != nullptr || d.pub.ctrl != nullptr || d.wait.ctrl != nullptr))
+        t = {256, 256};
+    Route r;
+    r.t = t;
+    if (d.bm != 0 || d.bn != 0 || d.wait.ctrl != nullptr || d.tail_act != nullptr || d.epi_act != nullptr) return r;
+    StreamKPlan pl;
+    if (d.streamk && !ForceSimple() && PlanStreamK(d.M, d.N, d.K, pl) &&
+        (d.pub.ctrl == nullptr || SplitPubOk(d.M, relay_rows)) && d.sk_ws != nullptr && d.sk_cnt != nullptr &&
+        d.sk_ws_bytes >= pl.WsBytes() && d.sk_cnt_len >= pl.tiles && (d.norm_y == nullptr || pl.G <= CuCount())) {
+        r.split = pl;
+    } else if (forced == nullptr && d.order_rows == 0 && OnePieceRelay(d.M, d.N, d.K, relay_rows, pl)) {
+        r.split = pl;
+    }
+    return r;
+}
+
+}  // namespace
+
 void GemmLaunch(const GemmDesc &d, hipStream_t stream)
 {
     if (d.K % 8 != 0) throw std::runtime_error("gemm: K must be a multiple of 8");
@@ -1672,26 +1726,8 @@ void GemmLaunch(const GemmDesc &d, hipStream_t stream)
         p.rn_spins = d.norm_max_spins > 0 ? d.norm_max_spins : kDefaultMaxSpins;
     }
     if (p.wait.ctrl != nullptr && p.wait.prod_rows <= 0) throw std::runtime_error("gemm: wait.prod_rows must be > 0");
-    const int relay_rows = d.pub.ctrl != nullptr ? d.pub.rows_per_tile : 0;
-    GemmTile t = GemmPickTile(d.M, d.N, relay_rows, d.coresident, d.K);
-    if (const char *e = std::getenv("KR_GEMM_TILE")) {
-        // tile sweep override "BMxBN" (measurement aid; bits are unchanged)
-        int bm = 0, bn = 0;
-        if (std::sscanf(e, "%dx%d", &bm, &bn) == 2 && (relay_rows == 0 || relay_rows % bm == 0)) t = {bm, bn};
-    }
-    if (d.bm > 0) {
-        // a forced M tile pairs with the widest N tile built for it
-        t.bm = d.bm;
-        t.bn = d.bn > 0 ? d.bn : 256;
-    } else if (d.bn > 0) {
-        t.bn = d.bn;
-    }
-    if (t.bm < 0) throw std::runtime_error("gemm: relay tile rows must be a multiple of 64");
-    // 192x256 runs only on the staged 8-wave kernel; elsewhere 256x256 (the
-    // same MFMA and K order: the same bits)
-    if (t.bm == 192 && (d.K % kPipeK != 0 || ForceSimple() || MainLoopMode() != 2 ||
-                        d.tail_act != nullptr || d.pub.ctrl != nullptr || d.wait.ctrl != nullptr))
-        t = {256, 256};
+    const Route route = RouteOf(d);
+    const GemmTile t = route.t;
     const bool bf = d.dtype == kBF16;
     if (d.dtype != kBF16 && d.dtype != kF16) throw std::runtime_error("gemm: dtype must be bf16 or f16");
     const int order = d.order_rows;
@@ -1700,32 +1736,18 @@ void GemmLaunch(const GemmDesc &d, hipStream_t stream)
         const int k = d.M / d.pub.rows_per_tile;
         tail = d.tail_tiles > 0 ? std::min(d.tail_tiles, k) : k;
     }
-    StreamKPlan skp;
-    const int rpt = d.pub.rows_per_tile;
-    if (d.streamk && d.wait.ctrl == nullptr && d.tail_act == nullptr && d.epi_act == nullptr && !ForceSimple() &&
-        d.bm == 0 && d.bn == 0 && PlanStreamK(d.M, d.N, d.K, skp) &&
-        (d.pub.ctrl == nullptr || SplitPubOk(d.M, rpt)) && d.sk_ws != nullptr && d.sk_cnt != nullptr &&
-        d.sk_ws_bytes >= skp.WsBytes() && d.sk_cnt_len >= skp.tiles &&
-        (d.norm_y == nullptr || skp.G <= CuCount())) {
-        p.sk_ws = static_cast<float *>(d.sk_ws);
-        p.sk_cnt = d.sk_cnt;
-        if (skp.bm == 128) {
-            bf ? LaunchSplit<kBF16, 128, 128>(p, skp, stream) : LaunchSplit<kF16, 128, 128>(p, skp, stream);
-            return;
+    if (route.split.G > 0) {
+        const StreamKPlan &pl = route.split;
+        if (pl.pmax > 1) {
+            p.sk_ws = static_cast<float *>(d.sk_ws);
+            p.sk_cnt = d.sk_cnt;
         }
-        if (skp.bm == 64) {
-            bf ? LaunchSplit<kBF16, 64, 128>(p, skp, stream) : LaunchSplit<kF16, 64, 128>(p, skp, stream);
-            return;
-        }
-        bf ? LaunchTyped<kBF16, 256, 256>(p, 0, 0, stream, &skp) : LaunchTyped<kF16, 256, 256>(p, 0, 0, stream, &skp);
-        return;
-    }
-    if (OnePieceRelay(d.M, d.N, d.K, relay_rows, skp) && d.bm == 0 && d.bn == 0 && std::getenv("KR_GEMM_TILE") == nullptr &&
-        d.wait.ctrl == nullptr && d.tail_act == nullptr && d.epi_act == nullptr && d.order_rows == 0) {
-        if (skp.bm == 128) {
-            bf ? LaunchSplit<kBF16, 128, 128>(p, skp, stream) : LaunchSplit<kF16, 128, 128>(p, skp, stream);
+        if (pl.bm == 128) {
+            bf ? LaunchSplit<kBF16, 128, 128>(p, pl, stream) : LaunchSplit<kF16, 128, 128>(p, pl, stream);
+        } else if (pl.bm == 64) {
+            bf ? LaunchSplit<kBF16, 64, 128>(p, pl, stream) : LaunchSplit<kF16, 64, 128>(p, pl, stream);
         } else {
-            bf ? LaunchSplit<kBF16, 64, 128>(p, skp, stream) : LaunchSplit<kF16, 64, 128>(p, skp, stream);
+            bf ? LaunchTyped<kBF16, 256, 256>(p, 0, 0, stream, &pl) : LaunchTyped<kF16, 256, 256>(p, 0, 0, stream, &pl);
         }
         return;
     }
@@ -1747,3 +1769,44 @@ void GemmLaunch(const GemmDesc &d, hipStream_t stream)
 }
 
 }  // namespace kr
+
+extern "C" int kr_gemm_route(int M, int N, int K, int64_t lda, int64_t ldb, int relay_rows, int ws, int norm, int *bm,
+                             int *bn, int *loop, int *pieces)
+{
+    using namespace kr;
+    try {
+        // stand-ins for device memory: the choice looks at their presence only
+        static int32_t mark;
+        GemmDesc d;
+        d.M = M;
+        d.N = N;
+        d.K = K;
+        d.lda = lda;
+        d.ldb = ldb;
+        if (relay_rows > 0) {
+            d.pub.ctrl = &mark;
+            d.pub.rows_per_tile = relay_rows;
+        }
+        if (norm != 0) d.norm_y = &mark;
+        size_t bytes = 0;
+        int counters = 0;
+        GemmStreamKNeeds(M, N, K, &bytes, &counters);
+        if (ws != 0 && bytes > 0) {
+            d.streamk = true;
+            d.sk_ws = &mark;
+            d.sk_ws_bytes = bytes;
+            d.sk_cnt = &mark;
+            d.sk_cnt_len = counters;
+        }
+        const Route r = RouteOf(d);
+        const bool split = r.split.G > 0;
+        *bm = split ? r.split.bm : r.t.bm;
+        *bn = split ? r.split.bn : r.t.bn;
+        *pieces = split ? r.split.pmax : 1;
+        *loop = int(split && r.split.bm < 256 ? GemmLoop::kDeep
+                                              : LoopOf(*bm, *bn, M, N, K, std::max(lda, ldb), split));
+        return 0;
+    } catch (const std::exception &) {
+        return 1;
+    }
+}

@@ -1,0 +1,32 @@
+"""The kernel the GEMM's dispatch takes for a shape, asked of the library on
+the CPU (kr_gemm_route launches nothing; without a device it counts 256 CUs)."""
+
+import ctypes
+from collections import namedtuple
+
+import pytest
+
+from kernrelay_amd import libapi
+
+LOOPS = ("simple", "ring", "deep", "staged", "wide")
+Route = namedtuple("Route", "bm bn loop pieces")
+
+
+def route(M, N, K, lda=None, ldb=None, relay_rows=0, ws=False, norm=False):
+    """None: the launch would be refused."""
+    fn = libapi.lib().kr_gemm_route
+    i32, i64, out = ctypes.c_int, ctypes.c_int64, ctypes.POINTER(ctypes.c_int)
+    fn.argtypes = [i32, i32, i32, i64, i64, i32, i32, i32, out, out, out, out]
+    v = [ctypes.c_int() for _ in range(4)]
+    rc = fn(M, N, K, K if lda is None else lda, K if ldb is None else ldb, relay_rows, int(ws), int(norm),
+            *(ctypes.byref(x) for x in v))
+    return None if rc else Route(v[0].value, v[1].value, LOOPS[v[2].value], v[3].value)
+
+
+@pytest.mark.parametrize("M,N", [(5, 24), (64, 4096), (200, 1536), (1024, 1024), (2048, 2048), (4096, 1000)])
+def test_one_stage_of_k_takes_the_small_tiles(M, N):
+    """K = 64 is one stage: a product with a CU for every 128x128 tile runs
+    them, not a 256-wide tile (2048x2048x64: 8.8 us against 5.7)."""
+    r = route(M, N, 64)
+    assert (r.bn, r.pieces) == (128, 1) and r.bm in (64, 128)
+    assert route(M, N, 64, ws=True) == r
