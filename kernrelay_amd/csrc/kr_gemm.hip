@@ -1038,10 +1038,17 @@ int CuCount()
     return v;
 }
 
-// Whether a launch of bm x bn tiles has at most one workgroup per CU.
-bool DeepGrid(int bm, int bn, int M, int N)
+// Whether a launch of bm x 128 tiles takes the deep ring: at most one
+// workgroup per CU, and for 128 rows a K of more than six stages. There its
+// four stages are filled at once and bring nothing to a K that ends with them,
+// while the kernel is slower to start (2048x1280, 160 tiles, two-stage ring
+// against deep: K 128 5.6 / 6.2 us, K 384 7.4 / 7.7, K 512 9.5 / 8.5;
+// 2048x2048, 256 tiles: K 192 6.3 / 6.9, K 384 8.7 / 8.2). 64 row tiles
+// are faster with it from K 64 on (1024x1024x128 5.6 -> 4.7).
+bool DeepGrid(int bm, int bn, int M, int N, int K)
 {
-    return ((M + bm - 1) / bm) * ((N + bn - 1) / bn) <= CuCount();
+    if (bm * bn >= 256 * 128 || bn != 128 || (bm == 128 && K <= 6 * kPipeK)) return false;
+    return int64_t((M + bm - 1) / bm) * ((N + bn - 1) / bn) <= CuCount();
 }
 
 // Whether the launch's 256-wide tiles run the wide loop: K of at least 32
@@ -1074,7 +1081,7 @@ GemmLoop LoopOf(int bm, int bn, int M, int N, int K, int64_t stride, bool sk)
     if (K % kPipeK != 0 || ForceSimple()) return GemmLoop::kSimple;
     if (!sk && WideLoop(bm, bn, M, N, K, stride)) return GemmLoop::kWide;
     if (bm == 256 && bn == 256 && (sk || PipeWaves() == 8)) return GemmLoop::kStaged;
-    if (bm * bn < 256 * 128 && bn == 128 && DeepGrid(bm, bn, M, N)) return GemmLoop::kDeep;
+    if (DeepGrid(bm, bn, M, N, K)) return GemmLoop::kDeep;
     return GemmLoop::kRing;
 }
 
