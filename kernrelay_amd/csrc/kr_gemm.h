@@ -124,8 +124,8 @@ enum class GemmLoop { kSimple, kRing, kDeep, kStaged, kWide };
 // What GemmLaunch runs for a product of these sizes and row strides
 // (elements): its tile, its loop (kr::GemmLoop) and the pieces of K each tile
 // is cut into (1: whole). relay_rows > 0: it releases relay tiles of that many
-// rows; ws: the caller gives the workspace GemmStreamKNeeds asks for; norm: with
-// the Add+RMSNorm relay consumer. Launches nothing. Non-zero: it would be
-// refused.
-extern "C" int kr_gemm_route(int M, int N, int K, int64_t lda, int64_t ldb, int relay_rows, int ws, int norm, int *bm,
+// rows; ws: the caller gives the workspace GemmStreamKNeeds asks for; use: 1 with
+// the Add+RMSNorm relay consumer, 2 with the SwiGLU epilogue. Launches nothing.
+// Non-zero: it would be refused.
+extern "C" int kr_gemm_route(int M, int N, int K, int64_t lda, int64_t ldb, int relay_rows, int ws, int use, int *bm,
                              int *bn, int *loop, int *pieces);

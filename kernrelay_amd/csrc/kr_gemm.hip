@@ -893,8 +893,13 @@ GemmKernel(GemmParams p)
         __syncthreads();
     }
 
-    if (p.epi_act != nullptr) {
-        StoreTileSwiglu<DT, BM, BN, kThreads>(p, acc, smem, m0, n0, wm, wn, lane);
+    // (SwigluTile: no launch asks 128-column tiles of this kernel for SwiGLU)
+    if constexpr (BN >= 256) {
+        if (p.epi_act != nullptr) {
+            StoreTileSwiglu<DT, BM, BN, kThreads>(p, acc, smem, m0, n0, wm, wn, lane);
+        } else {
+            StoreTile<DT, BM, BN, kThreads>(p, acc, smem, m0, n0, wm, wn, lane);
+        }
     } else {
         StoreTile<DT, BM, BN, kThreads>(p, acc, smem, m0, n0, wm, wn, lane);
     }
@@ -1083,6 +1088,17 @@ GemmLoop LoopOf(int bm, int bn, int M, int N, int K, int64_t stride, bool sk)
     if (bm == 256 && bn == 256 && (sk || PipeWaves() == 8)) return GemmLoop::kStaged;
     if (DeepGrid(bm, bn, M, N, K)) return GemmLoop::kDeep;
     return GemmLoop::kRing;
+}
+
+// The tile of a SwiGLU epilogue launch in place of t. The simple kernel and
+// the two-stage ring of the small tiles have no SwiGLU on 128 columns: its code
+// beside the plain epilogue cost every plain launch of them 0.1 to 0.4 us
+// (2048x1280x128 5.65 -> 5.80, 640x128x1000 17.4 -> 17.8). Such a launch takes
+// 256 columns.
+GemmTile SwigluTile(GemmTile t, GemmLoop loop)
+{
+    if (t.bn >= 256 || (loop != GemmLoop::kSimple && (t.bm * t.bn >= 256 * 128 || loop == GemmLoop::kDeep))) return t;
+    return {t.bm >= 256 ? 256 : 128, 256};
 }
 
 using GemmFn = void (*)(GemmParams);
@@ -1618,7 +1634,7 @@ Route RouteOf(const GemmDesc &d)
                         d.tail_act != nullptr || d.pub.ctrl != nullptr || d.wait.ctrl != nullptr))
         t = {256, 256};
     Route r;
-    r.t = t;
+    r.t = d.epi_act == nullptr ? t : SwigluTile(t, LoopOf(t.bm, t.bn, d.M, d.N, d.K, std::max(d.lda, d.ldb), false));
     if (d.bm != 0 || d.bn != 0 || d.wait.ctrl != nullptr || d.tail_act != nullptr || d.epi_act != nullptr) return r;
     StreamKPlan pl;
     if (d.streamk && !ForceSimple() && PlanStreamK(d.M, d.N, d.K, pl) &&
@@ -1777,7 +1793,7 @@ void GemmLaunch(const GemmDesc &d, hipStream_t stream)
 
 }  // namespace kr
 
-extern "C" int kr_gemm_route(int M, int N, int K, int64_t lda, int64_t ldb, int relay_rows, int ws, int norm, int *bm,
+extern "C" int kr_gemm_route(int M, int N, int K, int64_t lda, int64_t ldb, int relay_rows, int ws, int use, int *bm,
                              int *bn, int *loop, int *pieces)
 {
     using namespace kr;
@@ -1794,7 +1810,8 @@ extern "C" int kr_gemm_route(int M, int N, int K, int64_t lda, int64_t ldb, int 
             d.pub.ctrl = &mark;
             d.pub.rows_per_tile = relay_rows;
         }
-        if (norm != 0) d.norm_y = &mark;
+        if (use == 1) d.norm_y = &mark;
+        if (use == 2) d.epi_act = &mark;
         size_t bytes = 0;
         int counters = 0;
         GemmStreamKNeeds(M, N, K, &bytes, &counters);

@@ -12,13 +12,13 @@ LOOPS = ("simple", "ring", "deep", "staged", "wide")
 Route = namedtuple("Route", "bm bn loop pieces")
 
 
-def route(M, N, K, lda=None, ldb=None, relay_rows=0, ws=False, norm=False):
+def route(M, N, K, lda=None, ldb=None, relay_rows=0, ws=False, norm=False, swiglu=False):
     """None: the launch would be refused."""
     fn = libapi.lib().kr_gemm_route
     i32, i64, out = ctypes.c_int, ctypes.c_int64, ctypes.POINTER(ctypes.c_int)
     fn.argtypes = [i32, i32, i32, i64, i64, i32, i32, i32, out, out, out, out]
     v = [ctypes.c_int() for _ in range(4)]
-    rc = fn(M, N, K, K if lda is None else lda, K if ldb is None else ldb, relay_rows, int(ws), int(norm),
+    rc = fn(M, N, K, K if lda is None else lda, K if ldb is None else ldb, relay_rows, int(ws), 1 if norm else 2 * swiglu,
             *(ctypes.byref(x) for x in v))
     return None if rc else Route(v[0].value, v[1].value, LOOPS[v[2].value], v[3].value)
 
@@ -40,3 +40,17 @@ def test_short_k_keeps_the_two_stage_ring_of_128_row_tiles(M, N, K, loop):
     6.9 us against 6.3); 64 row tiles take it at any K."""
     assert route(M, N, K).loop == loop
     assert route(M, N, K, relay_rows=M // 4).loop == loop
+
+
+@pytest.mark.parametrize("M", [1, 37, 64, 65, 128, 200, 640, 1024, 2048, 4097])
+@pytest.mark.parametrize("N", [16, 272, 2176, 9728])
+@pytest.mark.parametrize("K", [64, 72, 256, 896, 904, 4096])
+def test_swiglu_tiles_have_the_epilogue(M, N, K):
+    """SwiGLU on 128 columns is built for the deep ring and the 256x128 tiles;
+    the simple kernel and the two-stage ring of the small tiles are built
+    without it (2% of every plain launch of the simple kernel)."""
+    r = route(M, N, K, swiglu=True)
+    assert r.bn == 256 or r.loop == "deep" or (r.bm == 256 and r.loop != "simple")
+    plain = route(M, N, K)
+    if plain.bn == 256 or plain.loop == "deep":
+        assert r == plain

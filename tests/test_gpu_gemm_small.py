@@ -81,8 +81,10 @@ def test_tiles_bit_exact(gpu, M, N, K, dt, bias):
     check(y, x, w, b)
 
 
-# the SwiGLU epilogue on 128-column tiles
-@pytest.mark.parametrize("M,cols,K", [(1, 8, 64), (37, 4864, 896), (200, 136, 896), (200, 12288, 4096)])
+# the SwiGLU epilogue on 128-column tiles, and where they are built without it
+# (K of one to six stages on more than 256 of the 64-row tiles, K no multiple of 64)
+@pytest.mark.parametrize("M,cols,K", [(1, 8, 64), (37, 4864, 896), (200, 136, 896), (200, 12288, 4096),
+                                      (1111, 1024, 256), (65, 72, 904)])
 def test_swiglu_small_tiles(gpu, M, cols, K):
     announce("gemm swiglu %dx%dx%d" % (M, cols, K))
     x, w, _ = make(M, 2 * cols, K, BF, False, 7)
