@@ -1059,20 +1059,36 @@ bool DeepGrid(int bm, int bn, int M, int N, int K)
 // Whether the launch's 256-wide tiles run the wide loop: K of at least 32
 // stages (its 4-wave prologue and epilogue, one wave per SIMD, cost more than
 // the 8-wave kernel's: 16384x2048x1024 71 -> 74 us), and workgroups for three
-// quarters of the CUs (with fewer the other loops were as fast or faster:
-// 2048x3584x3584 in 256x256 tiles 79 against 82 us, 1024x3584x3584 in
-// 256x128 48.6 against 49.6; full: 8192^3 789 -> 750, 4096x24576x4096 629 ->
-// 611, 2048x4096x12288 in 256x128 tiles 176 -> 163).
+// quarters of the CUs in 256x128 and 128x256 tiles (1024x3584x3584, 112 tiles,
+// 48.6 against 49.6 us; 1536x4096x4096, 192 tiles, 52.5 -> 51.1;
+// 2048x4096x12288, 256 tiles, 176 -> 167).
+// For 256x256 tiles, whose two-stage ring asks for a stage's data no earlier
+// than the stage before it, only where the 8-wave loop measured slower:
+// * four fifths of the CUs (8-wave / wide, us: 192 tiles 2048x6144x4096 85.5 /
+//   89, 16384x520x2048 45 / 47; 208 tiles 4096x3328x4096 90 / 87; 256
+//   tiles 4096x4096x8192 204 / 190);
+// * operands that come from the 256 MB Infinity Cache rather than HBM: all of
+//   them together (4096x3584: K 16384, 252 MB, 383 / 370; K 18944, 291 MB, 434 /
+//   467; 4096^2x16384, 268 MB, 409 / 460; 16384x1024: K 6144, 214 MB, 156 /
+//   149; K 8192, 285 MB, 212 / 220), or, over more than one round of
+//   workgroups, A in half of it (8192x8192: K 8192, A 134 MB, 801 / 754; K
+//   14336, A 235 MB, 1422 / 1451; 8192x4096x12288, A 201 MB, 602 / 617;
+//   4096x12288: K 16384, A 134 MB, 1211 / 1194; K 18944, A 155 MB, 1383 / 1412);
+// * no Add+RMSNorm consumer: its rows take 8 waves per workgroup faster
+//   (4096x3584x3584 108 / 113, 4096x4096x12288 316 / 324).
 // Its tile rows are addressed by 32-bit byte offsets: `stride` (elements) must
 // keep 256 of them below 4 GB.
-bool WideLoop(int bm, int bn, int M, int N, int K, int64_t stride)
+bool WideLoop(int bm, int bn, int M, int N, int K, int64_t stride, bool norm)
 {
     if (stride >= (int64_t(1) << 23)) return false;
     if (K % kPipeK != 0 || K < 32 * kPipeK || ForceSimple() || MainLoopMode() != 2 || PipeWaves() != 8 ||
         PrefetchStages() != 0)
         return false;
-    if (bm * bn != 256 * 128 && bm * bn != 256 * 256) return false;
-    return int64_t((M + bm - 1) / bm) * ((N + bn - 1) / bn) * 4 >= int64_t(CuCount()) * 3;
+    const int64_t tiles = int64_t((M + bm - 1) / bm) * ((N + bn - 1) / bn), cus = CuCount();
+    if (bm * bn == 256 * 128) return tiles * 4 >= cus * 3;
+    if (bm != 256 || bn != 256 || norm || tiles * 5 < cus * 4) return false;
+    constexpr int64_t kCache = int64_t(256) << 20;  // bytes
+    return 2 * int64_t(K) * (int64_t(M) + N) < kCache || (tiles > cus && 4 * int64_t(K) * M <= kCache);
 }
 
 // The loop a launch of bm x bn tiles runs over K: the simple kernel where
@@ -1080,11 +1096,11 @@ bool WideLoop(int bm, int bn, int M, int N, int K, int64_t stride)
 // (stream-K or data-parallel) unless KR_GEMM_WAVES=4; the wide loop for
 // 256-wide tiles with K long enough; the deep ring for a small tile whose
 // grid has at most one workgroup per CU; the 4-wave ring for the others.
-GemmLoop LoopOf(int bm, int bn, int M, int N, int K, int64_t stride, bool sk)
+GemmLoop LoopOf(int bm, int bn, int M, int N, int K, int64_t stride, bool sk, bool norm)
 {
     if (bm == 192) return GemmLoop::kStaged;
     if (K % kPipeK != 0 || ForceSimple()) return GemmLoop::kSimple;
-    if (!sk && WideLoop(bm, bn, M, N, K, stride)) return GemmLoop::kWide;
+    if (!sk && WideLoop(bm, bn, M, N, K, stride, norm)) return GemmLoop::kWide;
     if (bm == 256 && bn == 256 && (sk || PipeWaves() == 8)) return GemmLoop::kStaged;
     if (DeepGrid(bm, bn, M, N, K)) return GemmLoop::kDeep;
     return GemmLoop::kRing;
@@ -1105,9 +1121,9 @@ using GemmFn = void (*)(GemmParams);
 
 // The kernel of LoopOf's choice, and its block size.
 template <int DT, int BM, int BN>
-GemmFn PickGemmKernel(int M, int N, int K, int64_t stride, bool sk, int &threads)
+GemmFn PickGemmKernel(int M, int N, int K, int64_t stride, bool sk, bool norm, int &threads)
 {
-    [[maybe_unused]] const GemmLoop loop = LoopOf(BM, BN, M, N, K, stride, sk);
+    [[maybe_unused]] const GemmLoop loop = LoopOf(BM, BN, M, N, K, stride, sk, norm);
     if constexpr (BM == 192) {
         // 192x256: the 8-wave staged kernel only (GemmLaunch picks this tile
         // only where that kernel runs)
@@ -1150,13 +1166,13 @@ GemmFn PickGemmKernel(int M, int N, int K, int64_t stride, bool sk, int &threads
 // occupancy query on the exact instantiation (registers, LDS, waves);
 // cached per (dtype, tile, stream-K, loop).
 template <int DT, int BM, int BN>
-int GemmWgsPerCu(int M, int N, int K, int64_t stride, bool sk)
+int GemmWgsPerCu(int M, int N, int K, int64_t stride, bool sk, bool norm)
 {
     static int cache[2][5] = {};  // 0: not asked yet
-    int &c = cache[sk][int(LoopOf(BM, BN, M, N, K, stride, sk))];
+    int &c = cache[sk][int(LoopOf(BM, BN, M, N, K, stride, sk, norm))];
     if (c == 0) {
         int threads = 0;
-        const GemmFn fn = PickGemmKernel<DT, BM, BN>(M, N, K, stride, sk, threads);
+        const GemmFn fn = PickGemmKernel<DT, BM, BN>(M, N, K, stride, sk, norm, threads);
         int n = 0;
         Check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void *>(fn), threads, 0),
               "gemm occupancy");
@@ -1166,12 +1182,12 @@ int GemmWgsPerCu(int M, int N, int K, int64_t stride, bool sk)
     return c;
 }
 
-int GemmWgsPerCu(int dt, int bm, int bn, int M, int N, int K, int64_t stride, bool sk)
+int GemmWgsPerCu(int dt, int bm, int bn, int M, int N, int K, int64_t stride, bool sk, bool norm)
 {
     const bool bf = dt == kBF16;
 #define KR_OCC_CASE(BM_, BN_) \
-    if (bm == BM_ && bn == BN_) return bf ? GemmWgsPerCu<kBF16, BM_, BN_>(M, N, K, stride, sk) \
-                                                  : GemmWgsPerCu<kF16, BM_, BN_>(M, N, K, stride, sk);
+    if (bm == BM_ && bn == BN_) return bf ? GemmWgsPerCu<kBF16, BM_, BN_>(M, N, K, stride, sk, norm) \
+                                                  : GemmWgsPerCu<kF16, BM_, BN_>(M, N, K, stride, sk, norm);
     KR_OCC_CASE(256, 256)
     KR_OCC_CASE(192, 256)
     KR_OCC_CASE(256, 128)
@@ -1193,10 +1209,10 @@ int GemmWgsPerCu(int dt, int bm, int bn, int M, int N, int K, int64_t stride, bo
 bool NormRelayResident(int dt, int bm, int bn, int M, int N, int K, int rows_per_tile, int sk_wgs)
 {
     if (sk_wgs > 0 && bm < 256) return sk_wgs <= CuCount();  // GemmSplitKernel: one per CU
-    if (sk_wgs > 0) return sk_wgs <= CuCount() * GemmWgsPerCu(dt, 256, 256, M, N, K, K, true);
+    if (sk_wgs > 0) return sk_wgs <= CuCount() * GemmWgsPerCu(dt, 256, 256, M, N, K, K, true, true);
     if (rows_per_tile <= 0 || rows_per_tile % bm != 0 || M % rows_per_tile != 0) return false;
     const int per = (rows_per_tile / bm) * ((N + bn - 1) / bn);
-    return per <= CuCount() * GemmWgsPerCu(dt, bm, bn, M, N, K, K, false);
+    return per <= CuCount() * GemmWgsPerCu(dt, bm, bn, M, N, K, K, false, true);
 }
 
 // Estimated time (us) of a 256x256 split in S pieces (the last one sums all
@@ -1421,7 +1437,8 @@ void LaunchTyped(const GemmParams &base, int order_rows, int tail_tiles, hipStre
         // a grid resident as a whole releases every tile at about the same
         // time whatever the order: keep the grouped raster (square patches
         // per XCD, less operand traffic than relay-tile order)
-        if (sk == nullptr && p.gemm_wgs <= CuCount() * GemmWgsPerCu<DT, BM, BN>(p.M, p.N, p.K, std::max(p.lda, p.ldb), false)) p.order_rows = 0;
+        if (sk == nullptr && p.gemm_wgs <= CuCount() * GemmWgsPerCu<DT, BM, BN>(p.M, p.N, p.K, std::max(p.lda, p.ldb), false, true))
+            p.order_rows = 0;
     }
     if (sk != nullptr) {
         if (BM != 256 || BN != 256 || sk->tiles != p.gemm_wgs) throw std::logic_error("gemm: stream-K plan mismatch");
@@ -1436,7 +1453,7 @@ void LaunchTyped(const GemmParams &base, int order_rows, int tail_tiles, hipStre
     }
     const dim3 grid(grid_x);
     int threads = 0;
-    const GemmFn fn = PickGemmKernel<DT, BM, BN>(p.M, p.N, p.K, std::max(p.lda, p.ldb), sk != nullptr, threads);
+    const GemmFn fn = PickGemmKernel<DT, BM, BN>(p.M, p.N, p.K, std::max(p.lda, p.ldb), sk != nullptr, p.rn_y != nullptr, threads);
     void *args[] = {&p};
     Check(hipLaunchKernel(reinterpret_cast<const void *>(fn), grid, dim3(threads), args, 0, stream), "gemm launch");
 }
@@ -1634,7 +1651,7 @@ Route RouteOf(const GemmDesc &d)
                         d.tail_act != nullptr || d.pub.ctrl != nullptr || d.wait.ctrl != nullptr))
         t = {256, 256};
     Route r;
-    r.t = d.epi_act == nullptr ? t : SwigluTile(t, LoopOf(t.bm, t.bn, d.M, d.N, d.K, std::max(d.lda, d.ldb), false));
+    r.t = d.epi_act == nullptr ? t : SwigluTile(t, LoopOf(t.bm, t.bn, d.M, d.N, d.K, std::max(d.lda, d.ldb), false, false));
     if (d.bm != 0 || d.bn != 0 || d.wait.ctrl != nullptr || d.tail_act != nullptr || d.epi_act != nullptr) return r;
     StreamKPlan pl;
     if (d.streamk && !ForceSimple() && PlanStreamK(d.M, d.N, d.K, pl) &&
@@ -1828,7 +1845,7 @@ extern "C" int kr_gemm_route(int M, int N, int K, int64_t lda, int64_t ldb, int 
         *bn = split ? r.split.bn : r.t.bn;
         *pieces = split ? r.split.pmax : 1;
         *loop = int(split && r.split.bm < 256 ? GemmLoop::kDeep
-                                              : LoopOf(*bm, *bn, M, N, K, std::max(lda, ldb), split));
+                                              : LoopOf(*bm, *bn, M, N, K, std::max(lda, ldb), split, use == 1));
         return 0;
     } catch (const std::exception &) {
         return 1;

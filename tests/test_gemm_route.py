@@ -54,3 +54,18 @@ def test_swiglu_tiles_have_the_epilogue(M, N, K):
     plain = route(M, N, K)
     if plain.bn == 256 or plain.loop == "deep":
         assert r == plain
+
+
+@pytest.mark.parametrize("M,N,K,norm,loop", [
+    (4096, 3584, 16384, False, "wide"), (4096, 3584, 18944, False, "staged"), (4096, 4096, 12288, False, "wide"),
+    (4096, 4096, 16384, False, "staged"), (8192, 8192, 8192, False, "wide"), (8192, 8192, 14336, False, "staged"),
+    (8192, 4096, 12288, False, "staged"), (4096, 24576, 4096, False, "wide"), (16384, 520, 2048, False, "staged"),
+    (4096, 3584, 3584, False, "wide"), (4096, 3584, 3584, True, "staged"), (4096, 4096, 12288, True, "staged"),
+    (2048, 3584, 3584, False, "wide"), (2048, 3584, 3584, True, "wide"), (2048, 4096, 18944, False, "wide")])
+def test_wide_loop_where_it_is_the_faster(M, N, K, norm, loop):
+    """256x256 tiles run the wide loop over operands that the Infinity Cache
+    holds, with four fifths of the CUs and without the Add+RMSNorm consumer
+    (4096x3584x18944: 467 us against 434 in the 8-wave loop); the smaller
+    256-wide tiles run it at any K from 2048 on."""
+    r = route(M, N, K, relay_rows=M // 4 if norm else 0, norm=norm)
+    assert r.loop == loop and r.bm * r.bn >= 256 * 128, r
