@@ -46,7 +46,7 @@ enum {
 };
 
 /* Relay control blocks: 8 x int32 each, zero-initialised once by the owner
- * (layout: published, consumed, status, arrive, done, timed_out, -, -; the
+ * (layout: published, consumed, status, arrive, done, timed_out, left, -; the
  * first three words are the reference's kernels/kr_sync_common.h:10-15). */
 #define KR_CTRL_WORDS 8
 
@@ -132,7 +132,11 @@ int kr_op_gemm_swiglu_epilogue(int dtype, const void *A, int64_t lda, const void
  * y and sum are packed [M, N]; N in 136..4096, a multiple of 8. ws/counters
  * as for kr_op_gemm_streamk (NULL: data-parallel tiles). Fails (non-zero)
  * when a relay tile's producer workgroups cannot all be resident at once:
- * use smaller relay tiles. */
+ * use smaller relay tiles. Other work on the device may keep them from being
+ * placed together (another such call on another stream takes up to every
+ * CU): waits then end after about half a millisecond without the release and
+ * the workgroup that releases the tile works the rows left over, so the call
+ * gets slower and its results stay the same. */
 int kr_op_gemm_add_rmsnorm(int dtype, const void *A, int64_t lda, const void *Bt, int64_t ldb, void *C, int M,
                            int N, int K, const void *res, const void *gamma, void *y, void *sum, float *rstd_out,
                            float eps, const kr_pub *pub, uint32_t max_spins, void *ws, size_t ws_bytes,

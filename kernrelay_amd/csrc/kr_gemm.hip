@@ -299,17 +299,26 @@ __device__ void TailSwiglu(const GemmParams &p)
     }
 }
 
+// Finishers that release relay tile r of a split grid: of the row blocks that
+// touch it, in every column.
+__device__ __forceinline__ int RowTileArrivals(const GemmParams &p, int r, int bm)
+{
+    const int R = p.pub.rows_per_tile;
+    return ((min(r * R + R, p.M) - 1) / bm - r * R / bm + 1) * p.tiles_n;
+}
+
 // A split tile's finisher arrives on every relay tile that its rows m0 ..
-// m0 + bm - 1 touch; a relay tile is released by the finishers of the row
-// blocks that touch it, in every column.
-__device__ __forceinline__ void ArriveRows(const GemmParams &p, int m0, int bm)
+// m0 + bm - 1 touch. With `place`, LDS ints: its place in the arrival order of
+// the i-th goes to place[i].
+__device__ __forceinline__ void ArriveRows(const GemmParams &p, int m0, int bm, int *place = nullptr)
 {
     if (p.pub.ctrl == nullptr) return;
     RelayPub pub = p.pub;
-    const int R = pub.rows_per_tile;
-    for (int r = m0 / R; r * R < min(m0 + bm, p.M); ++r) {
-        pub.arrivals = ((min(r * R + R, p.M) - 1) / bm - r * R / bm + 1) * p.tiles_n;
-        RelayArrive(pub, r);
+    const int R = pub.rows_per_tile, r0 = m0 / R;
+    for (int r = r0; r * R < min(m0 + bm, p.M); ++r) {
+        pub.arrivals = RowTileArrivals(p, r, bm);
+        const int a = RelayArrive(pub, r);
+        if (place != nullptr && threadIdx.x == 0) place[r - r0] = a;
     }
 }
 
@@ -317,17 +326,21 @@ __device__ __forceinline__ void ArriveRows(const GemmParams &p, int m0, int bm)
 // The producer's own workgroups consume its released row tiles (the
 // reference's down -> Add+RMSNorm tile loop, exec/qwen_main.cpp:1274-1302,
 // without the all-reduce): a workgroup that has stored its C tile and arrived
-// on relay tile `tile`'s flag (as the tile's `worker`-th arrival) waits for
-// the tile's release (all of its producer workgroups have arrived), then
-// computes Add+RMSNorm for rows lo + worker*waves + wave, stepping by
-// workers*waves, one row per wave, RB rows' loads in flight at a time, with
-// the row code of the standalone row kernel. C is read at device scope
-// (written by other XCDs' workgroups of this launch). The last of the tile's
-// `workers` consumes the release (consumed + 1, status 1, or 2 when any wait
-// ran out of spins). Safe from deadlock because the launcher only asks for
-// it when the workgroups a tile waits for are resident together: the whole
-// grid, or (dispatched in order, relay tile after relay tile) one relay
-// tile's producers.
+// on the relay tile that its rows are in waits for the tile's release and then
+// computes Add+RMSNorm for its share of the tile's rows: as the s-th of
+// `workers` arrivals, rows lo + s*waves + wave, stepping by workers*waves, one
+// row per wave, RB rows' loads in flight at a time, with the row code of the
+// standalone row kernel. C is read at device scope (written by other XCDs'
+// workgroups of this launch). The last of the tile's `workers` consumes the
+// release (consumed + 1, status 1, or 2 when a wait ran past its spin bound).
+//
+// A workgroup that waits holds a CU that one of the tile's producers may need:
+// another such launch, or anything else on the device, can keep some of them
+// from being placed. So a wait ends after kNormPatience at the latest
+// without the release: the workgroups leave in the order in which they
+// arrived, and the one that releases the tile, which never waits, works the
+// shares of those that left after its own. Every placed workgroup ends by
+// itself, whatever else runs.
 template <int DT, int CPL, int RB>
 __device__ __forceinline__ void NormRows(const GemmParams &p, int lo, int hi, int first, int step)
 {
@@ -358,32 +371,74 @@ __device__ __forceinline__ void NormRows(const GemmParams &p, int lo, int hi, in
     }
 }
 
-template <int DT, int NW, int WPE>
-__device__ void NormTail(const GemmParams &p, int tile, int worker, int workers)
+// Spins (about 1 us each) after which a waiting workgroup leaves. The waits of
+// a grid that is placed as a whole are shorter: the last pieces' fix-up and
+// rows of C, tens of us.
+constexpr uint32_t kNormPatience = 512;
+constexpr int32_t kLeftReleased = INT32_MIN;  // set in the `left` word by the release
+
+// One lane: wait for the tile as its `place`-th arrival. False: it left.
+__device__ __forceinline__ bool NormWait(int32_t *flag, int place, uint32_t max_spins)
+{
+    const int32_t target = LoadRelaxed(flag + kOffConsumed) + 1;
+    uint32_t spins = 0;
+    while (LoadRelaxed(flag + kOffPublished) < target) {
+        if (++spins > min(max_spins, kNormPatience)) {
+            if (spins > max_spins) StoreRelaxed(flag + kOffTimedOut, 1);
+            int32_t left = place;  // all earlier ones have left, and the tile is not released
+            if (__hip_atomic_compare_exchange_strong(flag + kOffLeft, &left, place + 1, __ATOMIC_RELAXED,
+                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                return false;
+        }
+        __builtin_amdgcn_s_sleep(2);
+    }
+    return true;
+}
+
+// The part of the `place`-th arrival (thread 0 knows it) of relay tile
+// `tile`'s `workers`. slot: two LDS ints. NARROW: rows of up to two chunks per
+// lane in flight per wave.
+template <int DT, int NW, int WPE, int NARROW = WPE == 2 ? 4 : 8>
+__device__ __forceinline__ void NormTail(const GemmParams &p, int tile, int workers, int place, int *slot)
 {
     int32_t *flag = p.pub.ctrl + size_t(p.pub.flag0 + tile) * kWords;
-    if (threadIdx.x == 0) SpinOnTile(flag, flag, p.rn_spins);
+    if (threadIdx.x == 0) {
+        // (the last arrival released the tile)
+        if (place < workers - 1 && !NormWait(flag, place, p.rn_spins)) place = -1;
+        slot[0] = place;
+    }
     __syncthreads();
     const int R = p.pub.rows_per_tile;
     const int lo = tile * R, hi = min(lo + R, p.M);
-    const int first = worker * NW + int(threadIdx.x >> 6);
     const int step = workers * NW;
     // rows in flight per wave: what the registers hold without spilling
     // (WPE waves per SIMD share its 512 registers; loads land in the 256
     // architectural ones)
-    constexpr int RB4 = WPE == 2 ? 2 : 4;
-    constexpr int RB8 = WPE == 2 ? 1 : 2;
-    switch (p.rn_cpl) {
-        case 1: NormRows<DT, 1, RB4>(p, lo, hi, first, step); break;
-        case 2: NormRows<DT, 2, RB4>(p, lo, hi, first, step); break;
-        case 4: NormRows<DT, 4, RB4>(p, lo, hi, first, step); break;
-        default: NormRows<DT, 8, RB8>(p, lo, hi, first, step); break;
-    }
-    __syncthreads();
+    constexpr int CH = WPE == 2 ? 8 : 16;
+    int taken = 0;  // thread 0: shares left to this workgroup (known by the end of its own)
+    if (threadIdx.x == 0 && place == workers - 1)
+        taken = __hip_atomic_fetch_or(flag + kOffLeft, kLeftReleased, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // its own share (none: it left), then shares 0 .. taken - 1
+    int i = -1;
+    do {
+        const int share = i < 0 ? slot[0] : i;
+        const int first = share * NW + int(threadIdx.x >> 6);
+        if (share >= 0) {
+            switch (p.rn_cpl) {
+                case 1: NormRows<DT, 1, NARROW>(p, lo, hi, first, step); break;
+                case 2: NormRows<DT, 2, NARROW>(p, lo, hi, first, step); break;
+                case 4: NormRows<DT, 4, CH / 4>(p, lo, hi, first, step); break;
+                default: NormRows<DT, 8, CH / 8>(p, lo, hi, first, step); break;
+            }
+        }
+        if (threadIdx.x == 0) slot[1] = taken;
+        __syncthreads();
+    } while (++i < slot[1]);
     if (threadIdx.x == 0) {
         const int32_t a = __hip_atomic_fetch_add(flag + kOffDone, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (a == workers - 1) {
             StoreRelaxed(flag + kOffDone, 0);
+            StoreRelaxed(flag + kOffLeft, 0);
             const int32_t to = __hip_atomic_exchange(flag + kOffTimedOut, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             StoreRelaxed(flag + kOffConsumed, LoadRelaxed(flag + kOffConsumed) + 1);
             StoreRelaxed(flag + kOffStatus, to ? 2 : 1);
@@ -391,22 +446,20 @@ __device__ void NormTail(const GemmParams &p, int tile, int worker, int workers)
     }
 }
 
-// The Add+RMSNorm relay consumer of a split grid (G workgroups, all resident):
-// after its own pieces each workgroup takes a share of one relay tile (of
-// every G-th, should the tiles outnumber the workgroups). A share of every
-// tile in turn had each workgroup wait, load and count once per relay tile:
-// 768x4096x4096 in four relay tiles 65 us, 768x3584x18944 155.
+// The Add+RMSNorm relay consumer of a split tile's finisher, on every relay
+// tile that its rows touch. The other pieces' workgroups are done: the
+// finishers have a wave for every row of 64 and 128 row tiles, and two to eight
+// rows a wave in 256x256 ones (2048x3584x18944 in four relay tiles 251 ->
+// 255 us against all pieces on the rows, 2048x896x4864 56 -> 61).
+// NARROW 2: with more rows in flight the 256x256 split kernel spills. place: as
+// ArriveRows left it. (All workgroups on every relay tile in turn: 768x4096x4096
+// in four relay tiles 65 us, 768x3584x18944 155.)
 template <int DT, int NW, int WPE>
-__device__ __forceinline__ void NormTailShare(const GemmParams &p, int G)
+__device__ __forceinline__ void NormTailRows(const GemmParams &p, int m0, int bm, const int *place, int *slot)
 {
-    const int tiles = p.M / p.pub.rows_per_tile, b = int(blockIdx.x);
-    int t = b, first = b, next = b + 1;  // workgroups first .. next - 1 work on tile t
-    if (tiles < G) {
-        t = ((b + 1) * tiles - 1) / G;
-        first = t * G / tiles;
-        next = (t + 1) * G / tiles;
-    }
-    for (; t < tiles; t += G) NormTail<DT, NW, WPE>(p, t, b - first, next - first);
+    const int R = p.pub.rows_per_tile, r0 = m0 / R;
+    for (int r = r0; r * R < min(m0 + bm, p.M); ++r)
+        NormTail<DT, NW, WPE, 2>(p, r, RowTileArrivals(p, r, bm), place[r - r0], slot);
 }
 
 // The unary consumer's pass over the staged tile (after C's): y = f(C) with
@@ -905,8 +958,10 @@ GemmKernel(GemmParams p)
     }
     if (p.pub.ctrl != nullptr) {
         const int tile = m0 / p.pub.rows_per_tile;
-        const int a = RelayArriveIndexed(p.pub, tile, reinterpret_cast<int *>(smem));  // the tile stage is free
-        if (p.rn_y != nullptr) NormTail<DT, kThreads / 64, BM * BN >= 256 * 128 ? 1 : 2>(p, tile, a, p.pub.arrivals);
+        int *slot = reinterpret_cast<int *>(smem);  // the tile stage is free
+        const int a = RelayArriveIndexed(p.pub, tile, slot);
+        if (p.rn_y != nullptr)
+            NormTail<DT, kThreads / 64, BM * BN >= 256 * 128 ? 1 : 2>(p, tile, p.pub.arrivals, a, slot + 1);
     }
     RelayFinish(p.wait);
 }
@@ -1200,12 +1255,12 @@ int GemmWgsPerCu(int dt, int bm, int bn, int M, int N, int K, int64_t stride, bo
 }
 
 // The Add+RMSNorm relay consumer waits inside the producer's workgroups for
-// the other producer workgroups of its relay tile. Workgroups are dispatched
-// in id order (per XCD) and a relay tile's are consecutive ids, so the waits
-// always end when a relay tile's workgroups fit the device at once: then
-// every earlier tile's workgroups are resident or finished. A stream-K grid
-// must be resident as a whole. The device's slots come from the occupancy of
-// the kernel the launch runs.
+// the other producer workgroups of its relay tile, and is worth it where
+// those fit the device at once: workgroups are dispatched in id order (per
+// XCD) and a relay tile's are consecutive ids, so every earlier tile's are
+// resident or finished then; a split grid must fit as a whole. (Where the
+// device is not free for them the waits end by patience, NormTail.) The
+// device's slots come from the occupancy of the kernel the launch runs.
 bool NormRelayResident(int dt, int bm, int bn, int M, int N, int K, int rows_per_tile, int sk_wgs)
 {
     if (sk_wgs > 0 && bm < 256) return sk_wgs <= CuCount();  // GemmSplitKernel: one per CU
@@ -1377,6 +1432,10 @@ bool PlanStreamK(int M, int N, int K, StreamKPlan &pl)
     return true;
 }
 
+// With the Add+RMSNorm consumer a workgroup finishes one tile at most (not so in
+// the even spread of KR_GEMM_SK_WGS).
+bool SplitNormOk(const StreamKPlan &pl) { return pl.G <= CuCount() && pl.G == pl.tiles * pl.pmax; }
+
 // A split launch can release any relay tiles of whole 64-row blocks: a
 // finisher arrives on every relay tile its rows touch (ArriveRows), whether
 // they are whole row blocks or not.
@@ -1545,9 +1604,10 @@ bool GemmNormRelayFits(int M, int N, int K, int rows_per_tile, bool streamk_ws, 
 {
     if (AddRmsNormRowCpl(N) == 0 || rows_per_tile <= 0 || M % rows_per_tile != 0) return false;
     StreamKPlan skp;
-    if (streamk_ws && !ForceSimple() && PlanStreamK(M, N, K, skp) && SplitPubOk(M, rows_per_tile))
+    if (streamk_ws && !ForceSimple() && PlanStreamK(M, N, K, skp) && SplitPubOk(M, rows_per_tile) && SplitNormOk(skp))
         return NormRelayResident(dtype, skp.bm, skp.bn, M, N, K, rows_per_tile, skp.G);
-    if (OnePieceRelay(M, N, K, rows_per_tile, skp) && std::getenv("KR_GEMM_TILE") == nullptr) return true;
+    if (OnePieceRelay(M, N, K, rows_per_tile, skp) && std::getenv("KR_GEMM_TILE") == nullptr)
+        return NormRelayResident(dtype, skp.bm, skp.bn, M, N, K, rows_per_tile, skp.G);
     GemmTile t = GemmPickTile(M, N, rows_per_tile, false, K);
     if (const char *e = std::getenv("KR_GEMM_TILE")) {
         int bm = 0, bn = 0;
@@ -1656,7 +1716,7 @@ Route RouteOf(const GemmDesc &d)
     StreamKPlan pl;
     if (d.streamk && !ForceSimple() && PlanStreamK(d.M, d.N, d.K, pl) &&
         (d.pub.ctrl == nullptr || SplitPubOk(d.M, relay_rows)) && d.sk_ws != nullptr && d.sk_cnt != nullptr &&
-        d.sk_ws_bytes >= pl.WsBytes() && d.sk_cnt_len >= pl.tiles && (d.norm_y == nullptr || pl.G <= CuCount())) {
+        d.sk_ws_bytes >= pl.WsBytes() && d.sk_cnt_len >= pl.tiles && (d.norm_y == nullptr || SplitNormOk(pl))) {
         r.split = pl;
     } else if (forced == nullptr && d.order_rows == 0 && OnePieceRelay(d.M, d.N, d.K, relay_rows, pl)) {
         r.split = pl;

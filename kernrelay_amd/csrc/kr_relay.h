@@ -9,7 +9,9 @@
 //   [3] arrive     producer workgroup arrival ticket for the pending release
 //   [4] done       consumer workgroup completion ticket
 //   [5] timed_out  set by any consumer workgroup that exceeded its spin bound
-//   [6..7] unused
+//   [6] left       Add+RMSNorm run by the producer's workgroups: how many of
+//                  them gave up waiting, and whether the tile is released since
+//   [7] unused
 // A producer tile owns a *flag* block (words 0 and 3). Each consumer of that
 // tile owns a *state* block (words 1, 2, 4, 5). For a 1:1 edge both roles use
 // the same block, which is exactly the reference's [published, consumed,
@@ -42,6 +44,7 @@ constexpr int kOffStatus = 2;
 constexpr int kOffArrive = 3;
 constexpr int kOffDone = 4;
 constexpr int kOffTimedOut = 5;
+constexpr int kOffLeft = 6;
 
 constexpr uint32_t kDefaultMaxSpins = 1u << 22;
 
@@ -217,20 +220,23 @@ __device__ __forceinline__ void PutU16(void *p, uint16_t v, bool coherent)
 // Put* helpers (coherent = true). Each thread waits until its stores are
 // acknowledged at device scope, the barrier makes that true for the whole
 // workgroup, then one device-scope atomic arrives; the last arriving
-// workgroup releases the tile by bumping `published`.
-__device__ __forceinline__ void RelayArrive(const RelayPub &p, int tile)
+// workgroup releases the tile by bumping `published`. Returns this
+// workgroup's place in the arrival order (in thread 0).
+__device__ __forceinline__ int RelayArrive(const RelayPub &p, int tile)
 {
-    if (p.ctrl == nullptr) return;
+    int place = 0;
+    if (p.ctrl == nullptr) return place;
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this lane's stores are complete
     __syncthreads();
     if (threadIdx.x == 0) {
         int32_t *flag = p.ctrl + size_t(p.flag0 + tile) * kWords;
-        const int32_t t = __hip_atomic_fetch_add(flag + kOffArrive, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (t == p.arrivals - 1) {
+        place = __hip_atomic_fetch_add(flag + kOffArrive, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (place == p.arrivals - 1) {
             StoreRelaxed(flag + kOffArrive, 0);
             __hip_atomic_fetch_add(flag + kOffPublished, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
+    return place;
 }
 
 // RelayArrive that also returns to every thread this workgroup's place in

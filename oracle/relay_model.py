@@ -40,6 +40,7 @@ import time
 K_WORDS = 8
 OFF_PUBLISHED, OFF_CONSUMED, OFF_STATUS = 0, 1, 2
 OFF_ARRIVE, OFF_DONE, OFF_TIMED_OUT = 3, 4, 5
+OFF_LEFT = 6
 
 
 class Ctrl:
@@ -69,6 +70,13 @@ class Ctrl:
             old = self.w[b * K_WORDS + off]
             self.store(b, off, v)
             return old
+
+    def compare_exchange(self, b, off, want, v):
+        with self._lock:
+            if self.w[b * K_WORDS + off] != want:
+                return False
+            self.store(b, off, v)
+            return True
 
 
 def _yield(jitter):
@@ -234,65 +242,119 @@ def even_ranges(rows, groups):
 
 class InProducerRelay:
     """The relay consumer run by the producer's own workgroups (kr_gemm.hip
-    NormTail): each of a tile's ``arrivals`` workgroups writes its share of
-    the tile's rows, arrives with an indexed ticket (RelayArriveIndexed) —
-    the last one releases — then spins until ``published >= consumed + 1``,
-    reads the rows worker, worker + arrivals, ... of the whole tile (its
-    ticket is its worker index), and takes a done ticket; the last one
-    advances ``consumed`` and writes ``status``. One control block per tile
-    serves both roles, as a 1:1 edge does."""
+    NormTail): a tile has ``arrivals`` column tiles, each computed by
+    ``pieces`` workgroups of which the last one writes its rows and arrives
+    (the others are done); the last arrival releases the tile. Each arrival
+    spins until ``published >= consumed + 1``, reads its share of the whole
+    tile's rows (its place in the arrival order, + arrivals, ...), and takes a
+    done ticket; the last one advances ``consumed`` and writes ``status``. A
+    wait longer than ``patience`` spins ends: the workgroups leave in the
+    order in which they arrived, and the releasing one, which does not wait,
+    reads the shares of those that left. One control block per tile serves
+    both roles, as a 1:1 edge does."""
 
-    def __init__(self, tiles, rows, arrivals, max_spins=200000, mistake=None):
-        self.tiles, self.rows_per_tile, self.arrivals = tiles, rows, arrivals
-        self.max_spins, self.mistake = max_spins, mistake
+    RELEASED = 1 << 31
+
+    def __init__(self, tiles, rows, arrivals, max_spins=200000, mistake=None, pieces=1, patience=100000):
+        self.tiles, self.rows_per_tile, self.arrivals, self.pieces = tiles, rows, arrivals, pieces
+        self.max_spins, self.mistake, self.patience = max_spins, mistake, patience
         self.ctrl = Ctrl(tiles)
         self.rows = [-1] * (tiles * rows)
+        self.counters = Ctrl(-(-tiles * arrivals // K_WORDS))
+        self.leavers = 0
+
+    def _wait(self, t, place):
+        """NormWait. False: the workgroup left."""
+        c = self.ctrl
+        target = c.load(t, OFF_CONSUMED) + 1
+        spins = 0
+        while c.load(t, OFF_PUBLISHED) < target:
+            spins += 1
+            if self.mistake == "no_leaving":
+                if spins > self.max_spins:
+                    c.store(t, OFF_TIMED_OUT, 1)
+                    return True
+            elif spins > min(self.max_spins, self.patience):
+                if spins > self.max_spins:
+                    c.store(t, OFF_TIMED_OUT, 1)
+                if self.mistake == "leave_unseen" or c.compare_exchange(t, OFF_LEFT, place, place + 1):
+                    self.leavers += 1
+                    return False
+            time.sleep(0)
+        return True
 
     def workgroup(self, replay, t, w, jitter, seen, write_delay=0.0):
         c, base = self.ctrl, t * self.rows_per_tile
+        col = w % self.arrivals
         per = self.rows_per_tile // self.arrivals
-        lo = base + w * per
-        hi = base + (self.rows_per_tile if w == self.arrivals - 1 else (w + 1) * per)
+        lo = base + col * per
+        hi = base + (self.rows_per_tile if col == self.arrivals - 1 else (col + 1) * per)
         if write_delay:
             time.sleep(write_delay * w)
+        piece = divmod(t * self.arrivals + col, K_WORDS)
+        if self.pieces > 1:
+            if self.counters.fetch_add(*piece, 1) != self.pieces - 1:
+                return
+            self.counters.store(*piece, 0)
         for r in range(lo, hi):
             self.rows[r] = replay
             _yield(jitter)
-        worker = c.fetch_add(t, OFF_ARRIVE, 1)
-        if worker == self.arrivals - 1:
+        place, taken = c.fetch_add(t, OFF_ARRIVE, 1), 0
+        if place == self.arrivals - 1:
             c.store(t, OFF_ARRIVE, 0)
             c.fetch_add(t, OFF_PUBLISHED, 1)
-        if self.mistake != "no_wait":
-            target = c.load(t, OFF_CONSUMED) + 1
-            spins = 0
-            while c.load(t, OFF_PUBLISHED) < target:
-                spins += 1
-                if spins > self.max_spins:
-                    c.store(t, OFF_TIMED_OUT, 1)
-                    break
-                time.sleep(0)
-        for r in range(base + worker, base + self.rows_per_tile, self.arrivals):
-            seen.append((r, self.rows[r], replay))
-            _yield(jitter)
+            taken = c.fetch_add(t, OFF_LEFT, self.RELEASED)
+        elif self.mistake != "no_wait" and not self._wait(t, place):
+            place = -1
+        for share in ([place] if place >= 0 else []) + list(range(taken)):
+            for r in range(base + share, base + self.rows_per_tile, self.arrivals):
+                seen.append((r, self.rows[r], replay))
+                _yield(jitter)
         if c.fetch_add(t, OFF_DONE, 1) == self.arrivals - 1:
             c.store(t, OFF_DONE, 0)
+            c.store(t, OFF_LEFT, 0)
             to = c.exchange(t, OFF_TIMED_OUT, 0)
             c.store(t, OFF_CONSUMED, c.load(t, OFF_CONSUMED) + 1)
             c.store(t, OFF_STATUS, 2 if to else 1)
+
+    def jobs(self, replay, jitter, seen, write_delay=0.0, gate=None):
+        """Every workgroup as a thread, in dispatch order; with a gate, each
+        gives its place on the device back when it ends."""
+        def run(t, w):
+            self.workgroup(replay, t, w, jitter, seen, write_delay)
+            if gate is not None:
+                gate.release()
+
+        return [threading.Thread(target=run, args=(t, w)) for t in range(self.tiles)
+                for w in range(self.arrivals * self.pieces)]
 
     def replay(self, replay, jitter=0.2, write_delay=0.0):
         """All workgroups as threads, started in random order; with
         write_delay, workgroup w starts writing w * write_delay seconds late."""
         seen = []
-        ids = [(t, w) for t in range(self.tiles) for w in range(self.arrivals)]
-        random.shuffle(ids)
-        jobs = [threading.Thread(target=self.workgroup, args=(replay, t, w, jitter, seen, write_delay))
-                for t, w in ids]
+        jobs = self.jobs(replay, jitter, seen, write_delay)
+        random.shuffle(jobs)
         for th in jobs:
             th.start()
         for th in jobs:
             th.join()
         return seen
+
+
+def launch_together(relays, places, replay, jitter=0.0):
+    """One launch of every relay at once on a device with ``places`` for
+    workgroups: placed in turn, one of each launch at a time, and a
+    placed workgroup keeps its place until it ends. Returns what each read."""
+    gate = threading.Semaphore(places)
+    seen = [[] for _ in relays]
+    queues = [r.jobs(replay, jitter, s, gate=gate) for r, s in zip(relays, seen)]
+    order = [q[i] for i in range(max(map(len, queues))) for q in queues if i < len(q)]
+    for th in order:
+        gate.acquire()
+        th.start()
+    for th in order:
+        th.join()
+    return seen
 
 
 # ------------------------------------------ last-arrival fix-up of pieces ----

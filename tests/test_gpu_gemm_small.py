@@ -126,3 +126,75 @@ def test_relay_norm_odd_relay_tiles(gpu, M, N, K, k, streamk):
         blk = ctrl.cpu().reshape(k, ops.CTRL_WORDS)
         assert torch.all(blk[:, 0] == run) and torch.all(blk[:, 1] == run) and torch.all(blk[:, 2] == 1)
         assert torch.all(blk[:, 3:5] == 0)
+
+
+def norm_case(M, N, K, k, streamk, seed):
+    x, w, _ = make(M, N, K, BF, False, seed)
+    g = torch.Generator(device="cuda").manual_seed(seed + 1)
+    res, gamma = torch.randn(M, N, device="cuda", generator=g).to(BF), torch.ones(N, device="cuda").to(BF)
+    c, y, s, ref_c, ref_y, ref_s = (torch.empty(M, N, dtype=BF, device="cuda") for _ in range(6))
+    ws = cnt = None
+    if streamk:
+        nbytes, ncnt = ops.gemm_streamk_workspace(M, N, K)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+        cnt = torch.zeros(ncnt, dtype=torch.int32, device="cuda")
+        ops.gemm_streamk(x, w, ref_c, ws, cnt)
+    else:
+        ops.gemm(x, w, ref_c)
+    ops.rowop("add_rmsnorm", res, ref_y, x1=ref_c, gamma=gamma, sum_out=ref_s)
+    ctrl = torch.zeros(k * ops.CTRL_WORDS, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+
+    def run(stream=None, max_spins=0):
+        ops.gemm_add_rmsnorm(x, w, c, res, gamma, y, ops.make_pub(ctrl, 0, M // k), sum_out=s, ws=ws, counters=cnt,
+                             max_spins=max_spins, stream=stream)
+
+    def verify(runs, status):
+        assert torch.equal(c, ref_c) and torch.equal(y, ref_y) and torch.equal(s, ref_s)
+        blk = ctrl.cpu().reshape(k, ops.CTRL_WORDS)
+        assert torch.all(blk[:, 0] == runs) and torch.all(blk[:, 1] == runs) and torch.all(blk[:, 3:] == 0)
+        assert all(int(v) in status for v in blk[:, 2])
+        for t in (c, y, s):
+            t.zero_()
+
+    return run, verify
+
+
+# a spin bound of one or a few: most workgroups leave before the release and
+# the one that releases the tile works their rows (whole tiles in one piece
+# and two per CU, relay tiles that no row tile divides, split K in small and
+# 256x256 tiles with relay tiles above and below a row block)
+@pytest.mark.parametrize("M,N,K,k,streamk", [
+    (1024, 3584, 512, 4, False), (2048, 2048, 192, 2, False), (576, 4096, 512, 3, False), (256, 136, 72, 4, False),
+    (192, 896, 4864, 3, True), (128, 896, 4864, 2, True), (768, 3584, 18944, 4, True),
+    (2048, 896, 4864, 32, True), (2048, 896, 4864, 2, True), (4096, 4096, 256, 2, False)])
+def test_relay_norm_left_rows(gpu, M, N, K, k, streamk):
+    announce("gemm+add_rmsnorm leaving %dx%dx%d k=%d" % (M, N, K, k))
+    run, verify = norm_case(M, N, K, k, streamk, 11)
+    for n, spins in enumerate((1, 3, 20), 1):
+        run(max_spins=spins)
+        torch.cuda.synchronize()
+        verify(n, (1, 2))
+    run()
+    torch.cuda.synchronize()
+    verify(4, (1,))
+
+
+# launches on two streams that each take nearly every CU (224 workgroups, one
+# per CU): neither keeps the other from its end
+@pytest.mark.parametrize("M,N,K,k,streamk", [(1024, 3584, 512, 1, False), (1024, 3584, 512, 4, False),
+                                             (768, 3584, 18944, 4, True)])
+def test_relay_norm_two_streams(gpu, M, N, K, k, streamk):
+    announce("gemm+add_rmsnorm on two streams %dx%dx%d k=%d" % (M, N, K, k))
+    cases = [norm_case(M, N, K, k, streamk, seed) for seed in (12, 14)]
+    streams = [ops.QueueStream() for _ in cases]
+    try:
+        for _ in range(4):
+            for (run, _v), st in zip(cases, streams):
+                run(stream=st)
+        torch.cuda.synchronize()
+        for _run, verify in cases:
+            verify(4, (1,))
+    finally:
+        for st in streams:
+            st.close()

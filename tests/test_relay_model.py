@@ -184,6 +184,50 @@ def test_in_producer_relay_planted_mistake_no_wait():
     assert all(got == want for _, got, want in ok.replay(0, jitter=0.0, write_delay=2e-3))
 
 
+@pytest.mark.parametrize("pieces", [1, 3])
+@pytest.mark.parametrize("patience", [0, 3, 50])
+def test_in_producer_relay_leaving(pieces, patience):
+    """Workgroups that leave: every row is still read once per replay, after
+    it was written, and the tile's words are as without leaving."""
+    random.seed(50 + patience)
+    relay = RM.InProducerRelay(2, 24, 6, pieces=pieces, patience=patience)
+    for r in range(6):
+        seen = relay.replay(r)
+        assert sorted(row for row, _, _ in seen) == list(range(48))
+        assert all(got == want for _, got, want in seen)
+        for t in range(2):
+            assert relay.ctrl.load(t, RM.OFF_PUBLISHED) == relay.ctrl.load(t, RM.OFF_CONSUMED) == r + 1
+            assert relay.ctrl.load(t, RM.OFF_STATUS) == 1
+            assert all(relay.ctrl.load(t, off) == 0 for off in range(3, 8))
+    assert patience > 0 or relay.leavers > 0
+
+
+@pytest.mark.parametrize("pieces,places", [(1, 12), (2, 12)])
+def test_two_in_producer_relays_on_a_device_that_holds_one(pieces, places):
+    """Two launches placed in turn on a device with too few places for both:
+    each holds places that the other's producers need. They end by leaving,
+    rows whole; without leaving both run into their spin bound."""
+    relays = [RM.InProducerRelay(1, 32, 8, pieces=pieces, patience=40) for _ in range(2)]
+    for r in range(3):
+        for relay, seen in zip(relays, RM.launch_together(relays, places, r)):
+            assert sorted(row for row, _, _ in seen) == list(range(32))
+            assert all(got == want for _, got, want in seen)
+            assert relay.ctrl.load(0, RM.OFF_STATUS) == 1
+    assert sum(relay.leavers for relay in relays) > 0
+    held = [RM.InProducerRelay(1, 32, 8, pieces=pieces, max_spins=400, mistake="no_leaving") for _ in range(2)]
+    RM.launch_together(held, places, 0)
+    assert any(relay.ctrl.load(0, RM.OFF_STATUS) == 2 for relay in held)
+
+
+def test_in_producer_relay_planted_mistake_leaving_unseen():
+    """A workgroup that leaves without the releasing one seeing it takes its
+    rows with it."""
+    random.seed(9)
+    bad = RM.InProducerRelay(1, 32, 8, patience=0, mistake="leave_unseen")
+    seen = bad.replay(0, jitter=0.0, write_delay=2e-3)
+    assert sorted(row for row, _, _ in seen) != list(range(32))
+
+
 # ----------------------------------------- the last-arrival fix-up ----
 
 @pytest.mark.parametrize("pieces", [2, 4, 7])
