@@ -1111,6 +1111,10 @@ bool DeepGrid(int bm, int bn, int M, int N, int K)
     return int64_t((M + bm - 1) / bm) * ((N + bn - 1) / bn) <= CuCount();
 }
 
+// The larger of two row strides (elements); one that steps backwards counts
+// as the largest.
+int64_t RowSpan(int64_t lda, int64_t ldb) { return lda < 0 || ldb < 0 ? INT64_MAX : std::max(lda, ldb); }
+
 // Whether the launch's 256-wide tiles run the wide loop: K of at least 32
 // stages (its 4-wave prologue and epilogue, one wave per SIMD, cost more than
 // the 8-wave kernel's: 16384x2048x1024 71 -> 74 us), and workgroups for three
@@ -1131,8 +1135,8 @@ bool DeepGrid(int bm, int bn, int M, int N, int K)
 //   4096x12288: K 16384, A 134 MB, 1211 / 1194; K 18944, A 155 MB, 1383 / 1412);
 // * no Add+RMSNorm consumer: its rows take 8 waves per workgroup faster
 //   (4096x3584x3584 108 / 113, 4096x4096x12288 316 / 324).
-// Its tile rows are addressed by 32-bit byte offsets: `stride` (elements) must
-// keep 256 of them below 4 GB.
+// Its tile rows are addressed by unsigned 32-bit byte offsets: `stride`
+// (RowSpan) must keep 256 of them below 4 GB.
 bool WideLoop(int bm, int bn, int M, int N, int K, int64_t stride, bool norm)
 {
     if (stride >= (int64_t(1) << 23)) return false;
@@ -1496,7 +1500,7 @@ void LaunchTyped(const GemmParams &base, int order_rows, int tail_tiles, hipStre
         // a grid resident as a whole releases every tile at about the same
         // time whatever the order: keep the grouped raster (square patches
         // per XCD, less operand traffic than relay-tile order)
-        if (sk == nullptr && p.gemm_wgs <= CuCount() * GemmWgsPerCu<DT, BM, BN>(p.M, p.N, p.K, std::max(p.lda, p.ldb), false, true))
+        if (sk == nullptr && p.gemm_wgs <= CuCount() * GemmWgsPerCu<DT, BM, BN>(p.M, p.N, p.K, RowSpan(p.lda, p.ldb), false, true))
             p.order_rows = 0;
     }
     if (sk != nullptr) {
@@ -1512,7 +1516,7 @@ void LaunchTyped(const GemmParams &base, int order_rows, int tail_tiles, hipStre
     }
     const dim3 grid(grid_x);
     int threads = 0;
-    const GemmFn fn = PickGemmKernel<DT, BM, BN>(p.M, p.N, p.K, std::max(p.lda, p.ldb), sk != nullptr, p.rn_y != nullptr, threads);
+    const GemmFn fn = PickGemmKernel<DT, BM, BN>(p.M, p.N, p.K, RowSpan(p.lda, p.ldb), sk != nullptr, p.rn_y != nullptr, threads);
     void *args[] = {&p};
     Check(hipLaunchKernel(reinterpret_cast<const void *>(fn), grid, dim3(threads), args, 0, stream), "gemm launch");
 }
@@ -1711,7 +1715,7 @@ Route RouteOf(const GemmDesc &d)
                         d.tail_act != nullptr || d.pub.ctrl != nullptr || d.wait.ctrl != nullptr))
         t = {256, 256};
     Route r;
-    r.t = d.epi_act == nullptr ? t : SwigluTile(t, LoopOf(t.bm, t.bn, d.M, d.N, d.K, std::max(d.lda, d.ldb), false, false));
+    r.t = d.epi_act == nullptr ? t : SwigluTile(t, LoopOf(t.bm, t.bn, d.M, d.N, d.K, RowSpan(d.lda, d.ldb), false, false));
     if (d.bm != 0 || d.bn != 0 || d.wait.ctrl != nullptr || d.tail_act != nullptr || d.epi_act != nullptr) return r;
     StreamKPlan pl;
     if (d.streamk && !ForceSimple() && PlanStreamK(d.M, d.N, d.K, pl) &&
@@ -1905,7 +1909,7 @@ extern "C" int kr_gemm_route(int M, int N, int K, int64_t lda, int64_t ldb, int 
         *bn = split ? r.split.bn : r.t.bn;
         *pieces = split ? r.split.pmax : 1;
         *loop = int(split && r.split.bm < 256 ? GemmLoop::kDeep
-                                              : LoopOf(*bm, *bn, M, N, K, std::max(lda, ldb), split, use == 1));
+                                              : LoopOf(*bm, *bn, M, N, K, RowSpan(lda, ldb), split, use == 1));
         return 0;
     } catch (const std::exception &) {
         return 1;

@@ -69,3 +69,17 @@ def test_wide_loop_where_it_is_the_faster(M, N, K, norm, loop):
     256-wide tiles run it at any K from 2048 on."""
     r = route(M, N, K, relay_rows=M // 4 if norm else 0, norm=norm)
     assert r.loop == loop and r.bm * r.bn >= 256 * 128, r
+
+
+@pytest.mark.parametrize("lda,ldb,loop", [
+    (4096, 4096, "wide"), (4096, (1 << 23) - 8, "wide"), (0, 4096, "wide"), (1 << 23, 4096, "staged"),
+    (4096, 1 << 23, "staged"), (-4096, 4096, "staged"), (4096, -4096, "staged"), (-4096, -4096, "staged")])
+def test_wide_loop_row_strides(lda, ldb, loop):
+    """The wide loop's unsigned 32-bit row offsets hold neither a row that lies
+    4 GB ahead nor one that lies behind the tile's first: those would be read
+    out of bounds, and run the 64-bit addressing of the 8-wave loop."""
+    r = route(4096, 4096, 4096, lda=lda, ldb=ldb)
+    assert (r.bm, r.bn, r.loop) == (256, 256, loop)
+    for M, N in ((2048, 4096), (1024, 8192)):
+        r = route(M, N, 4096, lda=lda, ldb=ldb)
+        assert r.bm * r.bn == 256 * 128 and r.loop == ("wide" if loop == "wide" else "ring")
