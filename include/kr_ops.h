@@ -169,7 +169,9 @@ int kr_op_gemm_streamk(int dtype, const void *A, int64_t lda, const void *Bt, in
  * split needs more than the array holds fail with an error naming both
  * sizes. All calls on one GPU share the array: calls that may overlap in
  * time on one GPU (different streams, or host threads without ordering)
- * race and must not be issued. */
+ * race and must not be issued. Products with M or N below 256 or K below 2048
+ * take none of it: they run, and have the bits, as kr_op_gemm, and may
+ * overlap with anything. */
 int kr_op_gemm_streamk_noalloc(int dtype, const void *A, int64_t lda, const void *Bt, int64_t ldb, void *C,
                                int64_t ldc, const void *bias, int M, int N, int K, void *stream);
 

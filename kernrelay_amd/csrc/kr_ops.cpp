@@ -96,6 +96,12 @@ unsigned char *ScratchOnCurrentDevice()
     return static_cast<unsigned char *>(g_scratch[dev]);
 }
 
+// Products that may take the scratch: those that the 256x256 split covers (at
+// least one tile, two pieces of 16 stages). The smaller ones gain from a split
+// too (200x3584x3584 52 -> 19 us with a workspace), but calls of them on
+// several streams share nothing and may overlap.
+bool NoallocSplits(int M, int N, int K) { return M >= 256 && N >= 256 && K >= 2048; }
+
 // The counters start every call at zero (a fill kernel, not a memset, so the
 // call also works under graph capture).
 __global__ void ZeroCountersKernel(int32_t *c, int n)
@@ -235,7 +241,7 @@ int kr_op_gemm_streamk_noalloc(int dtype, const void *A, int64_t lda, const void
     return Guard([&] {
         size_t ws_bytes = 0;
         int counters = 0;
-        kr::GemmStreamKNeeds(M, N, K, &ws_bytes, &counters);
+        if (NoallocSplits(M, N, K)) kr::GemmStreamKNeeds(M, N, K, &ws_bytes, &counters);
         if (ws_bytes > kScratchPartialBytes || counters > kScratchCounters)
             throw std::runtime_error("gemm_streamk_noalloc: this shape's split needs " + std::to_string(ws_bytes) +
                                      " bytes of partials and " + std::to_string(counters) +

@@ -218,7 +218,8 @@ def gemm_streamk(A, Bt, C, ws, counters, bias=None, stream=None):
 
 def gemm_streamk_noalloc(A, Bt, C, bias=None, stream=None):
     """gemm_streamk with the library's own scratch (no workspace argument,
-    nothing allocated); raises for a split larger than the scratch."""
+    nothing allocated); raises for a split larger than the scratch. Products
+    with M or N below 256 or K below 2048 take none: as gemm."""
     M, K = A.shape
     N = Bt.shape[0]
     _check(_lib().kr_op_gemm_streamk_noalloc(_dt(A), _ptr(A), A.stride(0), _ptr(Bt), Bt.stride(0), _ptr(C),

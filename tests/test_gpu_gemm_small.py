@@ -198,3 +198,25 @@ def test_relay_norm_two_streams(gpu, M, N, K, k, streamk):
     finally:
         for st in streams:
             st.close()
+
+
+# products that the shared scratch of the allocation-free entry does not cover
+# (under a 256x256 tile, or fewer than two pieces of 16 stages): whole tiles, as
+# kr_op_gemm, also on two streams at once
+@pytest.mark.parametrize("M,N,K", [(200, 3584, 3584), (255, 896, 4864), (1000, 248, 4096), (300, 896, 1984)])
+def test_noalloc_small_takes_no_scratch(gpu, M, N, K):
+    announce("gemm streamk noalloc small %dx%dx%d" % (M, N, K))
+    assert ops.gemm_streamk_workspace(M, N, K)[0] > 0  # with a workspace it would split
+    cases = []
+    for seed in (16, 17):
+        x, w, b = make(M, N, K, BF, True, seed)
+        ref, y = torch.empty(M, N, dtype=BF, device="cuda"), torch.empty(M, N, dtype=BF, device="cuda")
+        ops.gemm(x, w, ref, bias=b)
+        cases.append((x, w, b, ref, y, torch.cuda.Stream()))
+    torch.cuda.synchronize()
+    for _ in range(8):
+        for x, w, b, _ref, y, st in cases:
+            ops.gemm_streamk_noalloc(x, w, y, bias=b, stream=st)
+    torch.cuda.synchronize()
+    for _x, _w, _b, ref, y, _st in cases:
+        assert torch.equal(y, ref)
