@@ -12,6 +12,7 @@ import torch
 
 from kernrelay_amd import ops
 from tests.conftest import announce
+from tests.test_gemm_route import route
 
 pytestmark = pytest.mark.gpu
 
@@ -62,8 +63,9 @@ def test_split_k_small(gpu, M, N, K, dt, bias):
     check(first, x, w, b)
 
 
-# deep-ring tiles with fewer stages than the ring, as many, and more; then the
-# wide loop's tiles (256x256, 256x128 and 128x256) with ragged edges
+# deep-ring tiles with fewer stages than the ring (one stage too), as many, and
+# more; then larger tiles with ragged rows, on the wide loop and on the staged
+# one (4097 columns: 192x256 tiles)
 @pytest.mark.parametrize("M,N,K,dt,bias", [
     (5, 24, 64, BF, False), (64, 128, 128, BF, True), (65, 129, 256, HF, False), (130, 260, 320, BF, True),
     (200, 896, 384, BF, False), (1024, 3584, 448, HF, False), (1111, 6144, 4096, HF, True),
@@ -71,6 +73,27 @@ def test_split_k_small(gpu, M, N, K, dt, bias):
 def test_tiles_bit_exact(gpu, M, N, K, dt, bias):
     announce("gemm tiles %dx%dx%d" % (M, N, K))
     x, w, b = make(M, N, K, dt, bias, 6)
+    pad = torch.full((M + 3, N + 16), 3.0, dtype=dt, device="cuda")
+    y = pad[:M, :N]
+    ops.gemm(x, w, y, bias=b)
+    ref = torch.empty(M, N, dtype=dt, device="cuda")
+    ops.gemm(x, w, ref, bias=b, bm=64)  # 64x256 tiles, two-stage ring
+    assert torch.equal(y, ref)
+    assert torch.all(pad[M:] == 3.0) and torch.all(pad[:, N:] == 3.0)
+    check(y, x, w, b)
+
+
+# the wide loop with ragged rows and columns in each of its tiles: the last tile's
+# rows of A and of B past the edge re-read the last row by their 32-bit offsets
+@pytest.mark.parametrize("M,N,K,dt,bias,tile", [
+    (4090, 3590, 2112, BF, True, (256, 256)), (3841, 4095, 2048, HF, False, (256, 256)),
+    (2041, 3465, 2112, BF, False, (256, 128)), (1793, 3969, 2048, HF, True, (256, 128)),
+    (515, 24571, 2048, BF, False, (128, 256)), (513, 24449, 2112, HF, True, (128, 256))])
+def test_wide_loop_ragged(gpu, M, N, K, dt, bias, tile):
+    announce("gemm wide loop %dx%dx%d" % (M, N, K))
+    r = route(M, N, K, lda=K + 24, ldb=K + 8)
+    assert ((r.bm, r.bn), r.loop) == (tile, "wide")
+    x, w, b = make(M, N, K, dt, bias, 9)
     pad = torch.full((M + 3, N + 16), 3.0, dtype=dt, device="cuda")
     y = pad[:M, :N]
     ops.gemm(x, w, y, bias=b)
