@@ -47,8 +47,8 @@ def log(msg):
 # what the same counter reads for a plain 512 MiB device copy; and rocprof's
 # MFMA utilisation of the same launches (SQ_VALU_MFMA_BUSY_CYCLES over
 # GRBM_GUI_ACTIVE x SIMDs, at the clock the card ran).
-GATE_UP_TRAFFIC_BYTES = (423154.0 * 2.0 + 75776.0 * 1.0) * 1024
-GATE_UP_MFMA_UTIL = 0.627
+GATE_UP_TRAFFIC_BYTES = (423236.0 * 2.0 + 75776.0 * 1.0) * 1024
+GATE_UP_MFMA_UTIL = 0.618
 GATE_UP_TRAFFIC_SOURCE = "profiles/gemm_gate_up_swiglu_2048x37888x3584.md"
 
 
@@ -72,7 +72,7 @@ def gemm_roofline(run, serial, S, N, K):
             "traffic": round(GATE_UP_TRAFFIC_BYTES) if measured else None,
             "traffic_algorithmic": 2 * (S * K + N * K + S * N // 2),
             "traffic_source": GATE_UP_TRAFFIC_SOURCE if measured else None,
-            "kernel": "GemmPipeKernel<bf16,256,256,8 waves> + its 192x256 wave-tail launch, gate/up projection "
+            "kernel": "GemmPipeKernel<bf16,256,256,4 waves,wide loop> + its 192x256 wave-tail launch, gate/up projection "
                       "%dx%dx%d, SwiGLU epilogue"
                       % (S, N, K),
             "avg_launch_us": round(avg_us, 2), "launches": int(run["gate_up_launches"]),
