@@ -14,6 +14,10 @@
  * Threading: one call at a time per process (the reference documents the
  * entry points as process-level, include/kernrelay.h:22-24). On HIP repeated
  * calls in one process are safe; concurrent calls are not supported.
+ *
+ * Kept between calls: up to four idle streams limited to CU masks, a hardware
+ * queue each, until the process ends. A process's first kr_plan_run or
+ * kr_qwen_run makes its two (14 ms with their end), later ones take them over.
  */
 #ifndef KERNRELAY_H
 #define KERNRELAY_H

@@ -22,10 +22,13 @@
 //   with (row>>1)&7, under which the 16 lanes of a fragment read (16
 //   consecutive rows, one chunk) hit distinct banks (0 conflict cycles
 //   measured by kernrelay_amd/probes/lds_banks.hip).
-// * Every variant walks K in the same order, and the two MFMA shapes give
-//   the same bits for the same K order, so a row of C is bit-identical
-//   whatever BM/BN or row range a launch covers: the split schedule is
-//   bit-exact against the unsplit one.
+// * Every data-parallel variant walks K in the same order, and the two MFMA
+//   shapes give the same bits for the same K order, so a row of C is
+//   bit-identical whatever BM/BN or row range a launch covers: the split
+//   schedule is bit-exact against the unsplit one. The split-K kernels
+//   (stream-K, GemmSplitKernel) sum their pieces of K in piece order: their bits
+//   follow the plan, a function of M, N and K alone, and differ from the
+//   data-parallel ones by the order of the fp32 sums.
 // * The MFMA is fed (B fragment, A fragment), so each block holds C^T: in a
 //   16x16 sub-block lane l owns row l % 16 and columns 4 (l / 16) .. + 3, in
 //   a 32x32 block row l % 32 and four runs of 4 columns.
@@ -1299,8 +1302,13 @@ double SmallTileUs(int bm, int S, int M, int N, int K)
 
 // Split plan of a small product (GemmSplitKernel): the cheapest of 64 and 128
 // row tiles in up to 16 pieces, taken when it beats the same tiles unsplit and
-// the 256x256 split `big` (its pieces; 0: none). Below 1920 rows only: longer
-// prompts keep the 256x256 plan and its workspace.
+// the 256x256 split `big` (its pieces; 0: none). Below 1920 rows only: from
+// there the plan, the workspace it reports and the bits are those of the
+// 256x256 split, which callers have been told. The line is not where the small
+// plan stops paying (us, 256x256 split / small plan / whole tiles: 2048x896x4864
+// 46.5 / 25.8 / 25.6, 2560x896x4864 47.8 / 31.9 / 31.8, 2048x1024x4096 43.2 /
+// 24.7 / 23.5, 2048x512x4096 41.8 / 19.1 / 21.6; 1919 rows of each take 24.8,
+// 23.4 and 17.3).
 bool PlanSplit(int M, int N, int K, int big, StreamKPlan &pl)
 {
     if (M >= 1920 || K % kPipeK != 0) return false;
@@ -1396,13 +1404,14 @@ int Split256Pieces(int M, int N, int tiles, int nk)
 // device's workgroup slots, or less than 90% with K of at least 256 stages
 // (16384), where two long pieces per 256x256 tile amortise the fix-up. The
 // last piece to finish sums all S partials alone, so short pieces lose to
-// that fix-up. Measured on MI355X with a warm activation: 2048x896x4864
-// data-parallel 67.1 us (best tile), 2 pieces 65.7, 4 pieces (19 stages)
-// 53.6, 8 pieces (9.5 stages) 78.2; 2048x896x896 with 2 pieces of 7 stages
-// 32.3 against 21.0. 2048x3584x18944 (the data-parallel 256x128 tiles fill
-// 87.5%): 226 us in two pieces of 148 stages against 248 us data-parallel in
-// the 7B prefill, on the 16x16x32 staged loop (KR_GEMM_SK_LONGK=0 keeps it
-// data-parallel). Spreading the iterations of every tile over all 256 CUs
+// that fix-up: 2048x896x4864 in 2 pieces 65.7 us, 4 pieces (19 stages) 53.6 (46.5
+// on the present loop), 8 pieces (9.5 stages) 78.2; 2048x896x896 with 2 pieces
+// of 7 stages 32.3 against 21.0. Both rules were fitted to the two-stage ring
+// and the staged loop: the whole tiles took 67.1 us for 2048x896x4864 (25.6 on the
+// deep ring now) and 248 for 2048x3584x18944 in the 7B prefill, against 226 in
+// two pieces of 148 stages. On the wide loop the whole 256x128 tiles take 225
+// us against the split's 231 alone and 257 against 260 in the prefill of one
+// card (KR_GEMM_SK_LONGK=0): the long-K split no longer gains there. Spreading the iterations of every tile over all 256 CUs
 // instead (pieces of uneven length at different K offsets, sharing no
 // operand lines) took 369 us for 2048x3584x18944. KR_GEMM_SK_WGS=G forces that
 // even spread over G workgroups (a measurement aid).

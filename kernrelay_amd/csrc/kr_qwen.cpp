@@ -661,10 +661,12 @@ private:
         a16(logits_, S * size_t(V_));
         rstd_.Alloc(S * 4);
         // Plain GEMMs split K over idle CUs where the GEMM planner finds an
-        // exact split (a data-parallel tiling that fills under 60% of the
-        // device and pieces of >= 16 K stages: the Qwen2.5-0.5B down
-        // projection, 4 pieces per tile; no 7B shape at seq 2048);
-        // KR_QWEN_SPLITK=0 turns it off. Every mode runs the same plan, so
+        // exact split (PlanStreamK): below 1920 rows most projections whose K
+        // of 2048 or more is cheaper in pieces on the small tiles; from there on
+        // those whose data-parallel tiling fills under 60% of the device, or
+        // 90% with K of 16384 or more (at 2048 rows the 0.5B down projection in
+        // four pieces per tile, the 7B one in two). KR_QWEN_SPLITK=0 turns it
+        // off. Every mode runs the same plan, so
         // the modes stay bit-identical. One workspace serves every plain GEMM
         // (they run one after another on the producer stream), sized for
         // whole-sequence and row-slice shapes; its tile counters start at

@@ -121,7 +121,8 @@ inline std::vector<uint32_t> ReservedCuMask(int num_cus, int per_xcd)
 
 // Idle CU-masked streams between runs. Making one (a hardware queue) takes 3.5
 // to 6 ms and destroying it 1.5 to 3, 14 ms for a run's pair: more than the
-// rest of a small schedule's run (1024x512x1024 with three consumers: 20 ms).
+// rest of a small schedule's run (1024x512x1024 with three consumers, a process's
+// second and later runs: 20 -> 5 to 7 ms; its first takes 37 either way).
 // A stream in use belongs to its run alone (taken out of the pool); it comes
 // back idle, outside any capture, and at most kMaxIdle wait here, the oldest
 // giving way. A stream that reports an error, in either direction, is dropped.
